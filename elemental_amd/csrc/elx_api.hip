@@ -52,6 +52,7 @@ std::map<int, DeviceInfo> g_info;
 std::map<std::pair<int, int>, Scratch> g_scratch;
 std::map<int, PanelSync> g_psync;
 std::map<int, PanelSync> g_xsync;  // one-XCD panel exchange areas (ordinary memory)
+std::map<int, RPanelSync> g_rsync;
 }  // namespace
 
 const DeviceInfo& device_info() {
@@ -176,6 +177,22 @@ elx_status_t xcd_sync_get(int max_groups, size_t slot_bytes, PanelSync** out) {
     return ELX_SUCCESS;
 }
 
+elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out) {
+    int dev = 0;
+    ELX_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_mu);
+    RPanelSync& rs = g_rsync[dev];
+    if (!rs.uarea)
+        ELX_HIP(hipExtMallocWithFlags(&rs.uarea, bytes, hipDeviceMallocUncached));
+    if (!rs.xarea) {
+        ELX_HIP(hipMalloc(&rs.xarea, bytes));
+        ELX_HIP(hipMemset(rs.xarea, 0, bytes));
+        ELX_HIP(hipDeviceSynchronize());
+    }
+    *out = &rs;
+    return ELX_SUCCESS;
+}
+
 // ---------------------------------------------------------------- kernel-class timing
 namespace {
 struct ProfRec {
@@ -247,6 +264,10 @@ elx_status_t release_all() {
         for (auto& kv : g_xsync)
             if (kv.second.slots) (void)hipFree(kv.second.slots);
         g_xsync.clear();
+        for (auto& kv : g_rsync) {
+            if (kv.second.xarea) (void)hipFree(kv.second.xarea);
+            kv.second.xarea = nullptr;
+        }
     }
     library_gemm_release();
     batched_release();

@@ -65,6 +65,8 @@ elx_status_t scratch_get(int slot, size_t bytes, void** out);
 constexpr int kSlotRuizWork = 64;
 // scratch slot of the full-pivoting LU's per-workgroup pivot candidates
 constexpr int kSlotFullPiv = 65;
+// scratch slot of the register panel's move list and row origins
+constexpr int kSlotRPanel = 66;
 
 // Per-device persistent state of the cooperative panel kernel's exchange area.
 struct PanelSync {
@@ -77,6 +79,16 @@ struct PanelSync {
 elx_status_t panel_sync_get(int max_groups, size_t slot_bytes, PanelSync** out);
 // The exchange area of the one-XCD panel: ordinary device memory (it stays in one XCD's L2).
 elx_status_t xcd_sync_get(int max_groups, size_t slot_bytes, PanelSync** out);
+
+// The register panel's exchange areas (lu_rpanel.hip): uncached memory (kept until the process
+// ends) and ordinary memory of the same layout. The launch counter never restarts, so a tag
+// left by an earlier launch is never taken for a current one.
+struct RPanelSync {
+    void* uarea = nullptr;
+    void* xarea = nullptr;
+    int64_t epoch = 0;
+};
+elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out);
 
 inline unsigned cdiv(i64 a, i64 b) { return (unsigned)((a + b - 1) / b); }
 
@@ -171,6 +183,13 @@ elx_status_t launch_lu_panel(hipStream_t s, i64 mp, i64 w, double* A, i64 lda, i
                              i64 goff, int2* pairs, int32_t* info);
 elx_status_t launch_lu_panel(hipStream_t s, i64 mp, i64 w, float* A, i64 lda, int32_t* dests,
                              i64 goff, int2* pairs, int32_t* info);
+
+// The panel with its rows in registers (lu_rpanel.hip), for heights that one XCD holds.
+bool rpanel_fits(i64 mp, i64 w);
+elx_status_t launch_rpanel(hipStream_t s, i64 mp, i64 w, double* A, i64 lda, int32_t* dests,
+                           i64 goff, int2* pairs, int32_t* info);
+elx_status_t launch_rpanel(hipStream_t s, i64 mp, i64 w, float* A, i64 lda, int32_t* dests,
+                           i64 goff, int2* pairs, int32_t* info);
 
 // The same panel for an fp32 matrix stored row by row: element (r, j) at A[r*lda + j]. With
 // xcd, the panel runs on the CUs of one XCD and exchanges its pivot candidates through that

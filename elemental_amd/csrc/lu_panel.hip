@@ -763,12 +763,14 @@ elx_status_t launch_lu_panel_f64(hipStream_t s, i64 mp, i64 w, double* A, i64 ld
 elx_status_t launch_lu_panel(hipStream_t s, i64 mp, i64 w, double* A, i64 lda, int32_t* dests,
                              i64 goff, int2* pairs, int32_t* info) {
     const bool xcd = xcd_panels_enabled() && xcd_fits<double>(mp, w);
+    if (!xcd && rpanel_fits(mp, w)) return launch_rpanel(s, mp, w, A, lda, dests, goff, pairs, info);
     return launch_panel<double>(s, mp, w, A, lda, 0, dests, goff, pairs, info, xcd);
 }
 
 elx_status_t launch_lu_panel(hipStream_t s, i64 mp, i64 w, float* A, i64 lda, int32_t* dests,
                              i64 goff, int2* pairs, int32_t* info) {
     const bool xcd = xcd_panels_enabled() && xcd_fits<float>(mp, w);
+    if (!xcd && rpanel_fits(mp, w)) return launch_rpanel(s, mp, w, A, lda, dests, goff, pairs, info);
     return launch_panel<float>(s, mp, w, A, lda, 0, dests, goff, pairs, info, xcd);
 }
 
