@@ -295,21 +295,30 @@ elx_status_t gate_slot(double** out) {
 
 namespace {
 
+constexpr i64 kChainRhs = 128;
+
 // General triangular solve: small-kernel diagonal blocks + MFMA GEMM updates. `stop` as in
 // the launchers: a recorded failure makes every step a no-op. allow_library false keeps the
-// updates on the hand-written GEMM (no library call, so nothing is allocated).
+// updates on the hand-written GEMM (no library call, so nothing is allocated). dot_order: a
+// single block's transposed backward solve in the reference BLAS's order.
 template <typename T>
 elx_status_t trsm_blocked(hipStream_t s, int side, int uplo, int orient, int diag, i64 m, i64 n,
                           T alpha, const T* A, i64 lda, T* B, i64 ldb,
-                          const int32_t* stop = nullptr, bool allow_library = true) {
+                          const int32_t* stop = nullptr, bool allow_library = true,
+                          bool dot_order = false) {
     if (m <= 0 || n <= 0) return ELX_SUCCESS;
     if (alpha != T(1))
         ELX_CHECK(launch_gemm(s, false, false, m, n, 0, T(0), (const T*)nullptr, 1,
                               (const T*)nullptr, 1, alpha, B, ldb, 0, stop, allow_library));
     const bool trans = (orient != kNormal);
     const i64 bs = 128;
+    // few right-hand sides: one chained launch instead of a diagonal solve and a GEMM per block
+    // (not where nothing may be allocated: its hand-off area is)
+    if (side == kLeft && allow_library && n <= kChainRhs && !(dot_order && m <= bs))
+        return launch_solve_chain(s, uplo, orient, diag, m, n, A, lda, B, ldb, stop);
     if (side == kLeft) {
-        if (m <= bs) return launch_trsm_small(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop);
+        if (m <= bs)
+            return launch_trsm_small(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop, dot_order);
         // M = op(A); forward when M is lower.
         const bool mlower = (uplo == kLower) != trans;
         const i64 nblk = (m + bs - 1) / bs;
@@ -343,7 +352,8 @@ elx_status_t trsm_blocked(hipStream_t s, int side, int uplo, int orient, int dia
         return ELX_SUCCESS;
     }
     // Right side: X op(A) = B, M = op(A) (n x n). Forward over column blocks when M is upper.
-    if (n <= bs) return launch_trsm_small(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop);
+    if (n <= bs)
+        return launch_trsm_small(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop, dot_order);
     const bool mupper = (uplo == kUpper) != trans;
     const i64 nblk = (n + bs - 1) / bs;
     for (i64 q = 0; q < nblk; ++q) {
@@ -702,7 +712,7 @@ elx_status_t trsm_api(void* stream, int side, int uplo, int orient, int diag, in
     ELX_ARG((side == kLeft || side == kRight) && (uplo == kLower || uplo == kUpper));
     ELX_ARG(orient >= 0 && orient <= 2 && (diag == kUnit || diag == kNonUnit));
     return trsm_blocked(static_cast<hipStream_t>(stream), side, uplo, orient, diag, m, n, alpha,
-                        dA, lda, dB, ldb);
+                        dA, lda, dB, ldb, nullptr, true, true);
 }
 
 template <typename T>

@@ -157,10 +157,10 @@ elx_status_t gate_slot(double** out);
 // factorization sequence (may be null); once it is non-zero the call changes nothing.
 elx_status_t launch_trsm_small(hipStream_t s, int side, int uplo, int orient, int diag, i64 m,
                                i64 n, const double* A, i64 lda, double* B, i64 ldb,
-                               const int32_t* stop = nullptr);
+                               const int32_t* stop = nullptr, bool dot_order = false);
 elx_status_t launch_trsm_small(hipStream_t s, int side, int uplo, int orient, int diag, i64 m,
                                i64 n, const float* A, i64 lda, float* B, i64 ldb,
-                               const int32_t* stop = nullptr);
+                               const int32_t* stop = nullptr, bool dot_order = false);
 // maxbits (may be null): the largest |entry| of the result is folded into *maxbits (bits of a
 // non-negative float, atomic max), for the exponent of the low-precision update that follows.
 elx_status_t launch_trsm_small_f32(hipStream_t s, int side, int uplo, int orient, int diag,

@@ -280,6 +280,10 @@ __global__ __launch_bounds__(NT) void rpanel_kernel(RArgs<T> p) {
                 int gw = g;
                 if constexpr (MULTI) {
                     if (wave == bw) {
+                        // the row lane cl just wrote, read by the others of this wave
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                         const uint32_t seq = p.seq_base + (uint32_t)c;
                         const bool have = bk.hi != 0;
                         const bool mine = lane >= s && lane <= WS;  // lane WS: the reciprocal
@@ -305,6 +309,7 @@ __global__ __launch_bounds__(NT) void rpanel_kernel(RArgs<T> p) {
                         bool got = lane >= p.G, ok = true;
                         int spins = 0;
                         while (true) {
+                            asm volatile("" ::: "memory");  // the load stays in the loop
                             if (!got) {
                                 const u4 r = l2 ? ld16<elx::xchg::kXcdLoad>(p.xarea, nunit, at)
                                                 : ld16(p.uarea, nunit, at);
@@ -330,6 +335,7 @@ __global__ __launch_bounds__(NT) void rpanel_kernel(RArgs<T> p) {
                             T v = T(0);
                             spins = 0;
                             while (true) {
+                                asm volatile("" ::: "memory");
                                 if (!in) {
                                     const u4 r = l2 ? ld16<elx::xchg::kXcdLoad>(p.xarea, nunit, rat)
                                                     : ld16(p.uarea, nunit, rat);

@@ -1,0 +1,269 @@
+// Triangular solves with an order <= 128 triangle and any number of vectors.
+#include <algorithm>
+#include <type_traits>
+
+#include "elx_common.hpp"
+#include "wave.hpp"
+
+using namespace elx::wv;
+
+namespace {
+
+// ---------------------------------------------------------------------------------------
+// Triangular solves M x = b for many independent vectors with an order <= 128 triangle.
+// Left side: the vectors are columns of B and M = op(A). Right side (X op(A) = B): the
+// vectors are rows of B and M = op(A)^T. Every entry is updated as the reference BLAS dtrsm
+// does: in forward and column-oriented backward substitution x_i -= M(i,j) x_j for j in turn,
+// one FMA each; division by the diagonal on the left side, multiplication by its reciprocal on
+// the right side.
+//
+// A wave solves 16 vectors in registers, with the backward forms run as forward ones on
+// reversed indices. The order is cut into 16-entry blocks: the block's 16 x 16 triangle is
+// solved with an entry per lane (x_k reaches the other 15 lanes of a vector by a DPP
+// broadcast), x goes through the wave's own LDS tile into operand layout, and the later blocks
+// are updated on the matrix cores, whose products are the same FMA chains in the same order,
+// so the results are the scalar code's bit for bit. No workgroup barrier; the triangle is read
+// straight from the caches in operand layout. What bounds it: per wave 8 dependent block solves
+// of 16 steps and 28 tile products, FP64 17-27 us (right side) and 11-24 us (left, unit
+// diagonal) from 64 to 16384 vectors, one wave per SIMD; with 16 lanes per vector, all 128 steps
+// dependent and 132 KB of LDS per 16 vectors, it took 52 us per 4096 vectors (240 us at 16256).
+//
+// maxbits (may be null): the largest |entry| written is folded into *maxbits (the bits of a
+// non-negative float, atomic max), for the exponent of a low-precision product that follows.
+// ---------------------------------------------------------------------------------------
+constexpr int TBLK = 16, TNB = 8;  // entries per block, blocks
+// FULL: order 128, no bounds on the order (the loads are then unconditional and go out together).
+template <typename T, bool RIGHT, bool UNIT, bool FULL>
+__global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const T* __restrict__ A,
+                                                         i64 lda, T* B, i64 ldb, int mtrans, int back,
+                                                         const int32_t* __restrict__ stop,
+                                                         unsigned* maxbits) {
+    typedef Mfma4<T> MF;
+    __shared__ T tiles[4][TBLK][TBLK + 1];
+    if (stop && *stop != 0) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l16 = lane & 15, kq = lane >> 4;
+    const i64 v0 = ((i64)blockIdx.x * 4 + wave) * TBLK;
+    if (v0 >= nvec) return;
+    T(*tile)[TBLK + 1] = tiles[wave];
+    // strides of M's logical rows and columns, and of an entry and a vector of B; the backward
+    // forms walk both from their ends
+    const i64 sgn = back ? -1 : 1;
+    const i64 si = sgn * (mtrans ? lda : 1), sj = sgn * (mtrans ? 1 : lda);
+    const i64 ei = sgn * (RIGHT ? ldb : 1), ev = RIGHT ? 1 : ldb;
+    const T* __restrict__ M0 = back ? A - (i64)(m - 1) * (si + sj) : A;
+    T* X0 = back ? B - (i64)(m - 1) * ei : B;
+    const T* __restrict__ Ml = M0 + l16 * si;            // row l16 of M
+    const T* __restrict__ Mk = Ml + kq * sj;             // and column kq: operand layout
+    const bool vin = v0 + l16 < nvec;
+    // the vectors: LEFT D(v, i), RIGHT D(i, v), so that lanes run along the contiguous index
+    typename MF::acc acc[TNB];
+#pragma unroll
+    for (int b = 0; b < TNB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = MF::row(kq, r);
+            const int i = TBLK * b + (RIGHT ? row : l16);
+            const i64 v = v0 + (RIGHT ? l16 : row);
+            acc[b][r] = ((FULL || i < m) && (RIGHT ? vin : v < nvec)) ? X0[i * ei + v * ev] : T(0);
+        }
+    float mx = 0.0f;
+    // a block's triangle (row l16), diagonal and the operands M(i, k) of the later blocks, loaded
+    // one block ahead
+    T mrow[2][TBLK], dgv[2], mop[2][TNB][4];
+    auto load = [&](auto bc) {
+        constexpr int b = decltype(bc)::value, p = b & 1;
+        const int ii = TBLK * b + l16;
+#pragma unroll
+        for (int k = 0; k < TBLK; ++k)
+            mrow[p][k] = (FULL || ii < m) && (FULL || k < l16) ? Ml[TBLK * b * si + (TBLK * b + k) * sj] : T(0);
+        dgv[p] = (!UNIT && (FULL || ii < m)) ? Ml[TBLK * b * si + ii * sj] : T(1);
+        static_for<b + 1, TNB>([&](auto nc) {
+            constexpr int nb = decltype(nc)::value;
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+                mop[p][nb][kk] = (FULL || TBLK * nb + l16 < m)
+                                     ? Mk[TBLK * nb * si + (TBLK * b + 4 * kk) * sj]
+                                     : T(0);
+        });
+    };
+    load(std::integral_constant<int, 0>{});
+    static_for<0, TNB>([&](auto bc) {
+        constexpr int b = decltype(bc)::value, p = b & 1;
+        if (FULL || TBLK * b < m) {
+            if constexpr (b + 1 < TNB) load(std::integral_constant<int, b + 1>{});
+            const T dg = (RIGHT && !UNIT) ? T(1) / dgv[p] : dgv[p];
+            // S(v, i): lane l16 holds entry i, register r vector MF::row(kq, r)
+            T x[4];
+            if (RIGHT) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tile[MF::row(kq, r)][l16] = acc[b][r];
+                wave_lds_sync();
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[r] = tile[l16][MF::row(kq, r)];
+                wave_lds_sync();
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[r] = acc[b][r];
+            }
+            // a lane's entry is final (but for its own diagonal) once the earlier ones are applied
+            static_for<0, TBLK>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const T dk = UNIT ? T(1) : row_bcast<k>(dg);
+                T xk[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    xk[r] = row_bcast<k>(x[r]);
+                    if (!UNIT) xk[r] = RIGHT ? xk[r] * dk : xk[r] / dk;
+                }
+                if (l16 > k) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[r] = __builtin_fma(-mrow[p][k], xk[r], x[r]);
+                }
+            });
+            if (!UNIT) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[r] = RIGHT ? x[r] * dg : x[r] / dg;
+            }
+            if (maxbits) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, (float)fabs(x[r]));
+            }
+            // into operand layout: X(v = l16, k = kq + 4 kk)
+            T xop[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) tile[MF::row(kq, r)][l16] = x[r];
+            wave_lds_sync();
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) xop[kk] = tile[l16][kq + 4 * kk];
+            wave_lds_sync();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = TBLK * b + (RIGHT ? kq + 4 * r : l16);
+                const i64 v = v0 + (RIGHT ? l16 : MF::row(kq, r));
+                if ((FULL || i < m) && (RIGHT ? vin : v < nvec)) X0[i * ei + v * ev] = RIGHT ? xop[r] : x[r];
+            }
+            // b_i -= m_ik x_k as fma(m_ik, -x_k, b_i): the same number
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) xop[kk] = -xop[kk];
+            static_for<b + 1, TNB>([&](auto nc) {
+                constexpr int nb = decltype(nc)::value;
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+                    acc[nb] = RIGHT ? MF::run(mop[p][nb][kk], xop[kk], acc[nb])
+                                    : MF::run(xop[kk], mop[p][nb][kk], acc[nb]);
+            });
+        }
+    });
+    if (maxbits) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+        if (lane == 0) atomicMax(maxbits, __float_as_uint(mx));
+    }
+}
+
+// The transposed backward forms as the reference BLAS computes them: each x_i a dot product in
+// ascending k from its nearest entry on, which is one dependent chain per vector. A thread per
+// vector, the vectors in LDS. Only a direct Trsm of order <= 128 asks for this order; the solves
+// of larger systems and of factored ones run their diagonal blocks through trsm_block_kernel.
+constexpr int DNT = 64;  // vectors per workgroup
+template <typename T>
+__global__ __launch_bounds__(DNT) void trsm_dot_kernel(int m, i64 nvec, const T* __restrict__ A, i64 lda,
+                                                       T* B, i64 ldb, int right, int unit,
+                                                       const int32_t* __restrict__ stop) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* xs = reinterpret_cast<T*>(smem_raw);  // xs[i * DNT + v]
+    if (stop && *stop != 0) return;
+    const int t = threadIdx.x;
+    const i64 v0 = (i64)blockIdx.x * DNT;
+    const int nv = (int)((nvec - v0) < DNT ? (nvec - v0) : DNT);
+    // a vector per lane (right) or down the columns (left): coalesced either way
+    for (int idx = t; idx < m * DNT; idx += DNT) {
+        const int i = right ? idx / DNT : idx % m, v = right ? idx % DNT : idx / m;
+        xs[i * DNT + v] = v < nv ? (right ? B[v0 + v + (i64)i * ldb] : B[i + (v0 + v) * ldb]) : T(0);
+    }
+    __syncthreads();
+    for (int i = m - 1; i >= 0; --i) {
+        const T* row = A + i * lda;  // M(i, k) = A(k, i)
+        T temp = xs[i * DNT + t];
+#pragma unroll 8
+        for (int k = i + 1; k < m; ++k) temp = __builtin_fma(-row[k], xs[k * DNT + t], temp);
+        if (!unit) temp = right ? temp * (T(1) / row[i]) : temp / row[i];
+        xs[i * DNT + t] = temp;
+    }
+    __syncthreads();
+    for (int idx = t; idx < m * DNT; idx += DNT) {
+        const int i = right ? idx / DNT : idx % m, v = right ? idx % DNT : idx / m;
+        if (v < nv) {
+            if (right) B[v0 + v + (i64)i * ldb] = xs[i * DNT + v];
+            else B[i + (v0 + v) * ldb] = xs[i * DNT + v];
+        }
+    }
+}
+
+}  // namespace
+
+namespace elx {
+
+// dot_order: the transposed backward forms in the reference BLAS's order (see trsm_dot_kernel).
+template <typename T>
+static elx_status_t trsm_small_impl(hipStream_t s, int side, int uplo, int orient, int diag,
+                                    i64 m, i64 n, const T* A, i64 lda, T* B, i64 ldb,
+                                    const int32_t* stop, bool dot_order, unsigned* maxbits = nullptr) {
+    if (m <= 0 || n <= 0) return ELX_SUCCESS;
+    const bool right = (side == kRight);
+    const i64 order = right ? n : m;
+    const i64 nvec = right ? m : n;
+    ELX_ARG(order <= 128);
+    const bool trans = (orient != kNormal);
+    const bool lower = (uplo == kLower);
+    // Left: M = op(A). Right: M = op(A)^T.
+    const bool mtrans = right ? !trans : trans;
+    const bool lower_eff = lower != mtrans;
+    const int unit = diag == kUnit ? 1 : 0, mt = mtrans ? 1 : 0;
+    ProfScope prof_(s, kKTrsm, (double)order * (double)order * (double)nvec);
+    if (!lower_eff && mtrans && dot_order) {
+        hipLaunchKernelGGL(trsm_dot_kernel<T>, dim3(cdiv(nvec, DNT)), dim3(DNT),
+                           sizeof(T) * (size_t)order * DNT, s, (int)order, nvec, A, lda, B, ldb, right ? 1 : 0, unit, stop);
+        ELX_HIP(hipGetLastError());
+        return ELX_SUCCESS;
+    }
+    const dim3 grid(cdiv(nvec, 4 * TBLK));
+    const int back = lower_eff ? 0 : 1;
+    auto go = [&](auto rt, auto ut) {
+        constexpr bool R = decltype(rt)::value, U = decltype(ut)::value;
+        if (order == TBLK * TNB)
+            hipLaunchKernelGGL((trsm_block_kernel<T, R, U, true>), grid, dim3(256), 0, s, (int)order,
+                               nvec, A, lda, B, ldb, mt, back, stop, maxbits);
+        else
+            hipLaunchKernelGGL((trsm_block_kernel<T, R, U, false>), grid, dim3(256), 0, s, (int)order,
+                               nvec, A, lda, B, ldb, mt, back, stop, maxbits);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (right) unit ? go(yes, yes) : go(yes, no);
+    else unit ? go(no, yes) : go(no, no);
+    ELX_HIP(hipGetLastError());
+    return ELX_SUCCESS;
+}
+
+elx_status_t launch_trsm_small(hipStream_t s, int side, int uplo, int orient, int diag, i64 m,
+                               i64 n, const double* A, i64 lda, double* B, i64 ldb,
+                               const int32_t* stop, bool dot_order) {
+    return trsm_small_impl<double>(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop, dot_order);
+}
+
+elx_status_t launch_trsm_small(hipStream_t s, int side, int uplo, int orient, int diag, i64 m,
+                               i64 n, const float* A, i64 lda, float* B, i64 ldb,
+                               const int32_t* stop, bool dot_order) {
+    return trsm_small_impl<float>(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop, dot_order);
+}
+
+elx_status_t launch_trsm_small_f32(hipStream_t s, int side, int uplo, int orient, int diag,
+                                   i64 m, i64 n, const float* A, i64 lda, float* B, i64 ldb,
+                                   unsigned* maxbits) {
+    return trsm_small_impl<float>(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, nullptr, false,
+                                  maxbits);
+}
+
+}  // namespace elx

@@ -1,0 +1,50 @@
+"""Diagonal-block kernels at the edges of their 16-entry blocks: the unblocked Cholesky (also where
+it stops, and beside infinities) and triangular solves of order <= 128, bit for bit the oracle's."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 48, 127, 128])
+def test_cholesky_block(dev, orc, n, dtype):
+    rng = np.random.default_rng(n)
+    G = rng.standard_normal((n, n))
+    H = (G @ G.T / n + np.eye(n)).astype(dtype)
+    H = np.tril(H) + np.tril(H, -1).T
+    cases = [("hpd", H)]
+    for j in sorted({0, n // 2, n - 1}):
+        S = H.copy()
+        S[j, j] = -1
+        cases.append((f"stops at {j}", S))
+    D = np.diag(np.arange(1, n + 1)).astype(dtype)  # exact zeros beside an infinity
+    D[n - 1, 0] = D[0, n - 1] = np.inf
+    cases.append(("inf beside zeros", D))
+    for name, A in cases:
+        for uplo in (0, 1):
+            print("[case]", n, dtype.__name__, name, uplo, flush=True)
+            F_ref, info_ref = orc.cholesky(A, uplo=uplo, bsize=128)
+            dA = dev.to_device(A)
+            info = dev.potrf(dA, uplo=uplo, nb=128)
+            tri = np.tril if uplo == 0 else np.triu
+            assert int(info.item()) == info_ref
+            assert np.array_equal(tri(dev.to_host(dA)), tri(F_ref), equal_nan=True)
+
+
+@pytest.mark.parametrize("side", [0, 1])
+def test_trsm_block_edges(dev, orc, side):
+    rng = np.random.default_rng(side)
+    for order in (15, 16, 31, 113, 127, 128):
+        for other in (4, 64, 65, 130):
+            for uplo in (0, 1):
+                for orient in (0, 1):
+                    for diag in (0, 1):
+                        print("[case]", side, order, other, uplo, orient, diag, flush=True)
+                        T = rng.standard_normal((order, order)) / np.sqrt(order) + 2 * np.eye(order)
+                        B = rng.standard_normal((order, other) if side == 0 else (other, order))
+                        dB = dev.to_device(B)
+                        dev.trsm(side, uplo, orient, diag, 1.0, dev.to_device(T), dB)
+                        ref = orc.trsm("LR"[side], "LU"[uplo], "NT"[orient], "NU"[diag], 1.0,
+                                       np.asfortranarray(T), np.asfortranarray(B))
+                        assert np.array_equal(dev.to_host(dB), ref)
