@@ -53,6 +53,7 @@ std::map<std::pair<int, int>, Scratch> g_scratch;
 std::map<int, PanelSync> g_psync;
 std::map<int, PanelSync> g_xsync;  // one-XCD panel exchange areas (ordinary memory)
 std::map<int, RPanelSync> g_rsync;
+std::map<int, ChainSync> g_csync;
 }  // namespace
 
 const DeviceInfo& device_info() {
@@ -186,6 +187,29 @@ elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out) {
         ELX_HIP(hipDeviceSynchronize());
     }
     *out = &rs;
+    return ELX_SUCCESS;
+}
+
+elx_status_t chain_sync_get(size_t bytes, ChainSync** out) {
+    int dev = 0;
+    ELX_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_mu);
+    ChainSync& cs = g_csync[dev];
+    if (!cs.ctrl) {
+        const uint32_t first[2] = {1u, 0u};  // epoch, workgroups finished
+        ELX_HIP(hipMalloc(&cs.ctrl, sizeof(first)));
+        ELX_HIP(hipMemcpy(cs.ctrl, first, sizeof(first), hipMemcpyHostToDevice));
+    }
+    if (cs.bytes < bytes) {
+        // the smaller area stays: queued launches may still use it, and uncached memory that a
+        // kernel has read is not freed
+        const size_t want = std::max<size_t>(std::max<size_t>(bytes, 2 * cs.bytes), (size_t)4 << 20);
+        void* area = nullptr;
+        ELX_HIP(hipExtMallocWithFlags(&area, want, hipDeviceMallocUncached));
+        cs.area = area;
+        cs.bytes = want;
+    }
+    *out = &cs;
     return ELX_SUCCESS;
 }
 

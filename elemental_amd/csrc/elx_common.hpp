@@ -90,6 +90,15 @@ struct RPanelSync {
 };
 elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out);
 
+// The hand-off area of the chained triangular solves (solve_chain.hip): uncached memory, grown by
+// doubling and kept until the process ends, and the launch epoch in device memory.
+struct ChainSync {
+    void* area = nullptr;
+    size_t bytes = 0;
+    void* ctrl = nullptr;
+};
+elx_status_t chain_sync_get(size_t bytes, ChainSync** out);
+
 inline unsigned cdiv(i64 a, i64 b) { return (unsigned)((a + b - 1) / b); }
 
 // Optional per-kernel-class timing with HIP events on the launching stream (off by default;
@@ -166,6 +175,13 @@ elx_status_t launch_trsm_small(hipStream_t s, int side, int uplo, int orient, in
 elx_status_t launch_trsm_small_f32(hipStream_t s, int side, int uplo, int orient, int diag,
                                    i64 m, i64 n, const float* A, i64 lda, float* B, i64 ldb,
                                    unsigned* maxbits = nullptr);
+
+// Left triangular solve of any order with few right-hand sides, one persistent launch per 16 of
+// them (solve_chain.hip).
+elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
+                                const double* A, i64 lda, double* B, i64 ldb, const int32_t* stop);
+elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
+                                const float* A, i64 lda, float* B, i64 ldb, const int32_t* stop);
 
 // General triangular solve (blocked by 128 with GEMM updates for larger triangles).
 elx_status_t dtrsm(hipStream_t s, int side, int uplo, int orient, int diag, i64 m, i64 n,

@@ -1,0 +1,75 @@
+"""The chained triangular solve (left side, order above 128, up to 128 right-hand sides): every
+orientation at the edges of its 128-row blocks, 16-row sub-blocks and groups of 16 right-hand
+sides. Substitution in any order satisfies |b - T x| <= gamma_n |T| |x| entry by entry
+(gamma_n ~ n u); evaluating that residual in FP64 costs as much again, hence the factor 2."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def residual_ok(T, x, b, u):
+    n = T.shape[0]
+    r = np.abs(b - T @ x)
+    return bool((r <= 2 * n * u * (np.abs(T) @ np.abs(x)) + np.finfo(np.float64).tiny).all())
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,nrhs,pad", [(129, 1, 0), (143, 16, 1), (256, 3, 2), (300, 17, 0),
+                                        (1000, 1, 3), (1153, 33, 1), (2200, 128, 0)])
+def test_all_orientations(dev, n, nrhs, pad, dtype):
+    rng = np.random.default_rng(n)
+    u = 2.0 ** -53 if dtype == np.float64 else 2.0 ** -24
+    M = (rng.standard_normal((n, n)) / np.sqrt(n)).astype(dtype)
+    M[np.arange(n), np.arange(n)] = (1.0 + rng.random(n)).astype(dtype)
+    buf = torch.zeros((n, n + pad), dtype=torch.from_numpy(M).dtype, device="cuda")
+    dM = buf.t()[:n]
+    dM.copy_(torch.from_numpy(M))
+    for uplo in (0, 1):
+        for orient in (0, 1):
+            for diag in (0, 1):
+                print("[case]", n, nrhs, pad, dtype.__name__, uplo, orient, diag, flush=True)
+                T = np.tril(M) if uplo == 0 else np.triu(M)
+                if diag == 1:
+                    T = T - np.diag(np.diag(T)) + np.eye(n, dtype=dtype)
+                T = (T if orient == 0 else T.T).astype(np.float64)
+                B = rng.standard_normal((n, nrhs)).astype(dtype)
+                dB = dev.to_device(B)
+                dev.trsm(0, uplo, orient, diag, 1.0, dM, dB)
+                assert residual_ok(T, dev.to_host(dB).astype(np.float64), B.astype(np.float64), u)
+
+
+def test_diagonal_out_of_the_quick_division_range(dev):
+    """Diagonal entries near the ends of the exponent range are divided by as they are."""
+    n = 200
+    rng = np.random.default_rng(1)
+    d = 2.0 ** rng.integers(-1000, 1000, n)
+    B = rng.standard_normal((n, 2))
+    dB = dev.to_device(B)
+    dev.trsm(0, 0, 0, 0, 1.0, dev.to_device(np.diag(d)), dB)
+    assert np.array_equal(dev.to_host(dB), B / d[:, None])
+
+
+def test_captured_solves_replay(dev):
+    """A captured lu::SolveAfter is replayed with new right-hand sides, eager solves between the
+    replays: every replay matches the eager result bit for bit."""
+    n = 700
+    rng = np.random.default_rng(2)
+    dA = dev.to_device(rng.standard_normal((n, n)))
+    d, info = dev.getrf(dA)
+    assert int(info.item()) == 0
+    dB = dev.to_device(rng.standard_normal((n, 3)))
+    dev.getrs(dA, d, dB)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        dev.getrs(dA, d, dB)
+    for _ in range(4):
+        B = rng.standard_normal((n, 3))
+        eager = dev.to_device(B)
+        dev.getrs(dA, d, eager)
+        dB.copy_(torch.from_numpy(B))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(dB, eager)
