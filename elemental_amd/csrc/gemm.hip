@@ -93,6 +93,51 @@ __device__ __forceinline__ void store_slab(T (*S)[BM + PAD], const T (&r)[8], T 
     }
 }
 
+// The tile of workgroup `bid`. Workgroups are dealt round-robin to the 8 XCDs, so each XCD takes a
+// contiguous run of a tile list that walks groups of 8 tile rows down the columns: tiles sharing A
+// rows and B columns share that XCD's L2. tri == 1 (2) lists the tiles on and below (above) the
+// diagonal of a square tile grid only: with the runs cut from the full grid, the last XCD's run
+// held nearly twice the mean number of live tiles and the launch waited for it.
+__device__ __forceinline__ bool tile_of(int bid, int tri, int tiles_m, int tiles_n, int& tm, int& tn) {
+    constexpr int GROUP = 8;
+    if (tri == 0) {
+        const int total = tiles_m * tiles_n, per_xcd = (total + 7) / 8;
+        const int lin = (bid % 8) * per_xcd + bid / 8;
+        if (lin >= total || bid / 8 >= per_xcd) return false;
+        const int group = lin / (GROUP * tiles_n), first_m = group * GROUP;
+        const int gsize = min(tiles_m - first_m, GROUP);
+        tm = first_m + (lin % (GROUP * tiles_n)) % gsize;
+        tn = (lin % (GROUP * tiles_n)) / gsize;
+        return true;
+    }
+    // group g: tile rows 8 g .. 8 g + 7, columns 0 .. 8 g + 7; 32 g^2 + 4 g tiles come before it
+    const int groups = (tiles_m + GROUP - 1) / GROUP, total = 32 * groups * groups + 4 * groups;
+    const int per_xcd = (total + 7) / 8, lin = (bid % 8) * per_xcd + bid / 8;
+    if (lin >= total || bid / 8 >= per_xcd) return false;
+    int g = (int)((sqrtf((float)lin * 8.0f + 1.0f) - 1.0f) * 0.0625f);
+    while (32 * (g + 1) * (g + 1) + 4 * (g + 1) <= lin) ++g;
+    while (32 * g * g + 4 * g > lin) --g;
+    int q = lin - (32 * g * g + 4 * g), r, c;
+    if (q < 64 * g) {  // left of the group's diagonal square
+        c = q / GROUP;
+        r = GROUP * g + q % GROUP;
+    } else {  // its lower triangle, column by column
+        q -= 64 * g;
+        int j = 0;
+        while (q >= GROUP - j) q -= GROUP - j++;
+        c = GROUP * g + j;
+        r = c + q;
+    }
+    if (r >= tiles_m) return false;
+    tm = tri == 1 ? r : c;
+    tn = tri == 1 ? c : r;
+    return true;
+}
+i64 tri_tiles(i64 tiles) {
+    const i64 groups = (tiles + 7) / 8;
+    return 32 * groups * groups + 4 * groups;
+}
+
 template <typename T, bool TA, bool TB>
 __global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alpha,
                                                   const T* __restrict__ A, i64 lda,
@@ -106,22 +151,9 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alph
     __shared__ T Bs[BK][BN + PAD];  // Bs[k][j] = op(B)(k0+k, n0+j)
     if (stop && *stop != 0) return;
 
-    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a contiguous run of
-    // tiles so that tiles sharing A rows / B columns share that XCD's L2.
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    const int lin = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-    if (lin >= total) return;
-    // Grouped ordering: walk 8 tile-rows at a time down the columns.
-    constexpr int GROUP = 8;
-    const int group = lin / (GROUP * tiles_n);
-    const int first_m = group * GROUP;
-    const int gsize = min(tiles_m - first_m, GROUP);
-    const int tm = first_m + (lin % (GROUP * tiles_n)) % gsize;
-    const int tn = (lin % (GROUP * tiles_n)) / gsize;
+    int tm, tn;
+    if (!tile_of((int)blockIdx.x, tri, tiles_m, tiles_n, tm, tn)) return;
     const i64 m0 = (i64)tm * BM, n0 = (i64)tn * BN;
-    if (tri == 1 && n0 > m0 + BM - 1) return;  // tile strictly above the diagonal
-    if (tri == 2 && m0 > n0 + BN - 1) return;  // tile strictly below the diagonal
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -295,8 +327,9 @@ __device__ __forceinline__ void dgemm_fast_tile(i64 M, i64 N, i64 K, double alph
     // the first slab's loads go out before C's, so that storing the slab waits for them alone
     // (loads complete in order) and C's 64 loads per thread stay in flight into the first steps
     gload(0);
-    if (FULL && fold && tri == 0) {
-        // the whole tile, no per-entry conditions (the LU's trailing update)
+    // a tile that the triangle does not cut carries no per-entry conditions
+    const bool whole = FULL && (tri == 0 || (tri == 1 ? m0 >= n0 + BN - 1 : n0 >= m0 + BM - 1));
+    if (whole && fold) {
         const double* c0 = C + m0 + wm + r16 + (n0 + wn + kq) * ldc;
 #pragma unroll
         for (int mi = 0; mi < 4; ++mi)
@@ -344,6 +377,16 @@ __device__ __forceinline__ void dgemm_fast_tile(i64 M, i64 N, i64 K, double alph
         __syncthreads();
         cur ^= 1;
     }
+    if (whole && fold) {
+        double* c0 = C + m0 + wm + r16 + (n0 + wn + kq) * ldc;
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) c0[mi * 16 + (ni * 16 + 4 * r) * ldc] = acc[mi][ni][r];
+        return;
+    }
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) {
         const i64 m = m0 + wm + mi * 16 + r16;
@@ -382,25 +425,22 @@ __global__ __launch_bounds__(NT, 2) void dgemm_fast_kernel(i64 M, i64 N, i64 K, 
                                                         i64 ldc, int tri, int tiles_m, int tiles_n,
                                                         const int32_t* __restrict__ stop) {
     if (stop && *stop != 0) return;
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    const int lin = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-    if (lin >= total) return;
-    constexpr int GROUP = 8;
-    const int group = lin / (GROUP * tiles_n);
-    const int first_m = group * GROUP;
-    const int gsize = min(tiles_m - first_m, GROUP);
-    const int tm = first_m + (lin % (GROUP * tiles_n)) % gsize;
-    const int tn = (lin % (GROUP * tiles_n)) / gsize;
+    int tm, tn;
+    if (FULL) {
+        if (!tile_of((int)blockIdx.x, tri, tiles_m, tiles_n, tm, tn)) return;
+    } else {
+        // the partial last tile row, then the partial last tile column
+        const int fm = (int)(M / BM), fn = (int)(N / BN), row = fm < tiles_m ? tiles_n : 0;
+        const int q = (int)blockIdx.x;
+        tm = q < row ? fm : q - row;
+        tn = q < row ? q : fn;
+    }
     const i64 m0 = (i64)tm * BM, n0 = (i64)tn * BN;
     if (tri == 1 && n0 > m0 + BM - 1) return;
     if (tri == 2 && m0 > n0 + BN - 1) return;
     // As[b][k][i] = sgn op(A)(m0+i, k0+k), Bs[b][k][j] = op(B)(k0+k, n0+j), double-buffered
     __shared__ __align__(16) double As[2][BK][BM + PAD];
     __shared__ __align__(16) double Bs[2][BK][BN + PAD];
-    // FULL: launched over the tiles inside C only; otherwise over every tile, the edge tiles
-    // done here and the full ones left to the FULL launch
-    if (!FULL && (m0 + BM <= M) && (n0 + BN <= N)) return;
     dgemm_fast_tile<TA, TB, FULL>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, m0, n0, As, Bs);
 }
 
@@ -442,6 +482,7 @@ elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T a
                        const int32_t* stop, bool allow_library) {
     using namespace elx;
     if (m <= 0 || n <= 0) return ELX_SUCCESS;
+    ELX_ARG(tri == 0 || m == n);
     if (k <= 0 || alpha == T(0)) {
         if (beta == T(1)) return ELX_SUCCESS;
         const unsigned blocks = (unsigned)std::min<i64>((m * n + 255) / 256, 65536);
@@ -493,10 +534,9 @@ elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T a
             const i64 fm = m / BM, fn = n / BN;
             const i64 tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
             ELX_ARG(tm * tn < (i64)1 << 30);
-            auto go = [&](auto full_tag, i64 gm, i64 gn) {
+            auto go = [&](auto full_tag, i64 gm, i64 gn, unsigned blocks) {
                 constexpr bool F = decltype(full_tag)::value;
                 if (gm <= 0 || gn <= 0) return;
-                const unsigned blocks = (unsigned)(((gm * gn + 7) / 8) * 8);
                 const int igm = (int)gm, ign = (int)gn;
                 if (!ta && !tb)
                     hipLaunchKernelGGL((dgemm_fast_kernel<false, false, F>), dim3(blocks), dim3(NT), 0,
@@ -511,8 +551,10 @@ elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T a
                     hipLaunchKernelGGL((dgemm_fast_kernel<true, true, F>), dim3(blocks), dim3(NT), 0,
                                        s, m, n, k, al, dA, lda, dB, ldb, be, dC, ldc, tri, igm, ign, stop);
             };
-            go(std::integral_constant<bool, true>{}, fm, fn);
-            if (fm != tm || fn != tn) go(std::integral_constant<bool, false>{}, tm, tn);
+            const i64 list = tri ? tri_tiles(fm) : fm * fn;
+            go(std::integral_constant<bool, true>{}, fm, fn, (unsigned)((list + 7) / 8 * 8));
+            const i64 edge = (fm < tm ? tn : 0) + (fn < tn ? fm : 0);
+            if (edge > 0) go(std::integral_constant<bool, false>{}, tm, tn, (unsigned)edge);
             ELX_HIP(hipGetLastError());
             return ELX_SUCCESS;
         }
@@ -520,7 +562,8 @@ elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T a
     const i64 tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
     ELX_ARG(tm * tn < (i64)1 << 30);
     ProfScope prof_(s, kKDgemm, flops);
-    const unsigned blocks = (unsigned)(((tm * tn + 7) / 8) * 8);
+    const i64 list = tri ? tri_tiles(tm) : tm * tn;
+    const unsigned blocks = (unsigned)((list + 7) / 8 * 8);
     const int itm = (int)tm, itn = (int)tn;
     if (!ta && !tb)
         hipLaunchKernelGGL((gemm_kernel<T, false, false>), dim3(blocks), dim3(NT), 0, s, m, n, k,
