@@ -29,6 +29,7 @@
 
 #include "elx_common.hpp"
 #include "exchange.hpp"
+#include "wave.hpp"
 
 namespace {
 
@@ -37,11 +38,10 @@ using elx::xchg::mix32;
 using elx::xchg::st16;
 using elx::xchg::u4;
 
-constexpr int NT = 512;                    // 8 waves: two per SIMD, 256 VGPRs each
-constexpr int NW = NT / 64;
+constexpr int NTMAX = 512;                 // 8 waves: two per SIMD, 256 VGPRs each
 constexpr int WS = 32;                     // columns per block
 constexpr int RPT = 2;                     // rows per thread (two named halves of the code)
-constexpr int RWG = NT * RPT;              // rows per workgroup
+constexpr int RWG = NTMAX * RPT;           // rows per workgroup
 constexpr int GMAX = 32;                   // workgroups (one XCD's CUs)
 constexpr int NC = WS / 8;                 // 8-column chunks of a row
 constexpr int WPANEL = 128;                // widest panel
@@ -181,8 +181,11 @@ __device__ __forceinline__ uint32_t xcc_id() {
 // double-buffered by column parity (a workgroup publishes column c + 2 only after it has read
 // every record of column c + 1, each of which was published after its writer had read column
 // c's row).
-template <typename T, bool MULTI>
+// NT: threads. A block of at most 128 (512) rows runs in 1 (4) waves: fewer waves to wait for at
+// the barriers and a SIMD of its own for each.
+template <typename T, bool MULTI, int NT>
 __global__ __launch_bounds__(NT) void rpanel_kernel(RArgs<T> p) {
+    constexpr int NW = NT / 64;
     __shared__ __align__(16) uint4 rec[2][NW];   // a wave's candidate: key, label
     __shared__ T rows[2][ROWLD];                 // the best candidate's row and reciprocal
     __shared__ T grow[2][ROWLD];                 // the winner's (MULTI)
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(NT) void rpanel_kernel(RArgs<T> p) {
 
     T a[RPT][WS];
     int lbl[RPT], org[RPT];
-    const i64 r0 = (i64)g * RWG + t;
+    const i64 r0 = (i64)g * (NT * RPT) + t;
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
         const i64 r = r0 + q * NT;
@@ -521,44 +524,54 @@ __global__ __launch_bounds__(256) void panel_solve_kernel(T* P, i64 lda, i64 mp,
         if (dst >= 0 && j0 + q < jend) D[dst + (i64)(j0 + q) * lda] = x[q];
 }
 
-// A22 -= L21 U12 inside the panel: rank 32, a row per thread, UC columns per workgroup. The
-// thread's 32 multipliers are loaded once (consecutive threads, consecutive rows); U12's entries
-// are the same for every thread and come through the scalar cache.
-constexpr int UC = 8;
+// A22 -= L21 U12 inside the panel: rank 32 on the matrix cores (bit for bit the FMA chain over k),
+// a 16 x 16 tile of A22 per wave, every operand loaded straight into its lane before the first
+// product. One memory latency and 8 products: at these sizes the launch is latency-bound (a row
+// per thread with U12 through the scalar cache took 6-13 us, this 4-9).
+constexpr int UR = 64, UC = 16;  // rows, columns per workgroup
 template <typename T>
 __global__ __launch_bounds__(256) void panel_update_kernel(const T* __restrict__ L, const T* __restrict__ U,
                                                            T* __restrict__ C, i64 lda, i64 rows, int cols,
                                                            const int32_t* __restrict__ done) {
+    typedef elx::wv::Mfma4<T> MF;
     const int steps = *done;
-    const i64 r = (i64)blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, kq = lane >> 4;
+    const i64 r = (i64)blockIdx.x * UR + wave * 16 + l16;
     const int j0 = (int)blockIdx.y * UC;
-    if (r >= rows || steps <= 0) return;
-    T l[WS];
+    if (steps <= 0) return;
+    const bool rin = r < rows, jin = j0 + l16 < cols;
+    T l[WS / 4], u[WS / 4];
 #pragma unroll
-    for (int k = 0; k < WS; ++k) l[k] = (k < steps) ? L[r + (i64)k * lda] : T(0);
-    T c[UC];
+    for (int kk = 0; kk < WS / 4; ++kk) {
+        const int k = 4 * kk + kq;
+        l[kk] = (rin && k < steps) ? L[r + (i64)k * lda] : T(0);
+        u[kk] = (jin && k < steps) ? U[k + (i64)(j0 + l16) * lda] : T(0);
+    }
+    // D(j, r): lanes run down the columns of A22
+    typename MF::acc c;
 #pragma unroll
-    for (int e = 0; e < UC; ++e) c[e] = (j0 + e < cols) ? C[r + (i64)(j0 + e) * lda] : T(0);
-    if (steps == WS && j0 + UC <= cols) {
+    for (int q = 0; q < 4; ++q) {
+        const int j = j0 + MF::row(kq, q);
+        c[q] = (rin && j < cols) ? C[r + (i64)j * lda] : T(0);
+    }
+    if (steps == WS) {
 #pragma unroll
-        for (int e = 0; e < UC; ++e) {
-            const T* u = U + (i64)(j0 + e) * lda;
-#pragma unroll
-            for (int k = 0; k < WS; ++k) c[e] = __builtin_fma(-l[k], u[k], c[e]);
-        }
+        for (int kk = 0; kk < WS / 4; ++kk) c = MF::run(u[kk], -l[kk], c);
     } else {
+        // a block that stopped: only its completed steps (a zero operand would meet infinities)
+        for (int k = 0; k < steps; ++k) {
 #pragma unroll
-        for (int e = 0; e < UC; ++e) {
-            if (j0 + e >= cols) break;
-            const T* u = U + (i64)(j0 + e) * lda;
-#pragma unroll
-            for (int k = 0; k < WS; ++k)
-                if (k < steps) c[e] = __builtin_fma(-l[k], u[k], c[e]);
+            for (int q = 0; q < 4; ++q) {
+                const int j = j0 + MF::row(kq, q);
+                if (rin && j < cols) c[q] = __builtin_fma(-L[r + (i64)k * lda], U[k + (i64)j * lda], c[q]);
+            }
         }
     }
 #pragma unroll
-    for (int e = 0; e < UC; ++e)
-        if (j0 + e < cols) C[r + (i64)(j0 + e) * lda] = c[e];
+    for (int q = 0; q < 4; ++q) {
+        const int j = j0 + MF::row(kq, q);
+        if (rin && j < cols) C[r + (i64)j * lda] = c[q];
+    }
 }
 
 template <typename T>
@@ -601,7 +614,12 @@ elx_status_t rpanel(hipStream_t s, i64 mp, i64 W, T* P, i64 lda, int32_t* dests,
         if (a.G == 1) {
             a.seq_base = 0;
             a.uarea = a.xarea = nullptr;
-            hipLaunchKernelGGL((rpanel_kernel<T, false>), dim3(1), dim3(NT), 0, s, a);
+            if (a.mp <= 64 * RPT)
+                hipLaunchKernelGGL((rpanel_kernel<T, false, 64>), dim3(1), dim3(64), 0, s, a);
+            else if (a.mp <= 256 * RPT)
+                hipLaunchKernelGGL((rpanel_kernel<T, false, 256>), dim3(1), dim3(256), 0, s, a);
+            else
+                hipLaunchKernelGGL((rpanel_kernel<T, false, NTMAX>), dim3(1), dim3(NTMAX), 0, s, a);
             ELX_HIP(hipGetLastError());
         } else {
             a.seq_base = (uint32_t)((++sync->epoch) * WS);
@@ -610,7 +628,7 @@ elx_status_t rpanel(hipStream_t s, i64 mp, i64 W, T* P, i64 lda, int32_t* dests,
             // an ordinary launch (a cooperative one costs 11 us before and after it on this
             // stream): at most one workgroup per CU of one XCD waits on others, each gets its
             // CU as soon as earlier work drains, and every wait is bounded
-            hipLaunchKernelGGL((rpanel_kernel<T, true>), dim3(8 * (unsigned)a.G), dim3(NT), 0, s, a);
+            hipLaunchKernelGGL((rpanel_kernel<T, true, NTMAX>), dim3(8 * (unsigned)a.G), dim3(NTMAX), 0, s, a);
             ELX_HIP(hipGetLastError());
         }
         const int nr = (int)(W - c0 - w);
@@ -625,7 +643,7 @@ elx_status_t rpanel(hipStream_t s, i64 mp, i64 W, T* P, i64 lda, int32_t* dests,
             const T* L = P + (c0 + w) + c0 * lda;
             T* C = P + (c0 + w) + (c0 + w) * lda;
             const T* U = P + c0 + (c0 + w) * lda;
-            hipLaunchKernelGGL(panel_update_kernel<T>, dim3((unsigned)((rows + 255) / 256), (nr + UC - 1) / UC),
+            hipLaunchKernelGGL(panel_update_kernel<T>, dim3((unsigned)((rows + UR - 1) / UR), (nr + UC - 1) / UC),
                                dim3(256), 0, s, L, U, C, lda, rows, nr, done);
             ELX_HIP(hipGetLastError());
         }
