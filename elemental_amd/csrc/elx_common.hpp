@@ -161,6 +161,16 @@ elx_status_t launch_gemm(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, f
 // Two device doubles per device for the coefficients of gated library calls.
 elx_status_t gate_slot(double** out);
 
+// The same for an update that gathers several 128-column panels, the first at column `from`: once
+// `stop` holds the failing column, only the panels completed before it are applied.
+elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, double alpha,
+                              const double* A, i64 lda, const double* B, i64 ldb, double beta,
+                              double* C, i64 ldc, int tri, const int32_t* stop, i64 from);
+elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, float alpha,
+                              const float* A, i64 lda, const float* B, i64 ldb, float beta, float* C,
+                              i64 ldc, int tri, const int32_t* stop, i64 from);
+bool gemm_library_selected();  // ELX_DGEMM=library
+
 // Small triangular solves for many independent vectors (triangle order <= 128).
 // side/uplo/orient/diag as in Elemental. B is m x n. `stop`: the info word of a
 // factorization sequence (may be null); once it is non-zero the call changes nothing.

@@ -54,7 +54,8 @@ struct Mfma<float> {
 // Loads of one BK-slab of op(A) (BM x BK) or op(B) (BK x BN) into 8 registers per thread.
 // "mn-contiguous" operands (op(A) = A, op(B) = B^T) have 128 contiguous entries per k;
 // "k-contiguous" operands (op(A) = A^T, op(B) = B) have 16 contiguous entries per m/n.
-template <bool KCONTIG, typename T>
+// FULL: the slab lies inside the operand.
+template <bool KCONTIG, bool FULL, typename T>
 __device__ __forceinline__ void load_slab(const T* __restrict__ P, i64 ld, i64 mn0,
                                           i64 MN, i64 k0, i64 K, T (&r)[8]) {
     const int t = threadIdx.x;
@@ -65,7 +66,7 @@ __device__ __forceinline__ void load_slab(const T* __restrict__ P, i64 ld, i64 m
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const i64 i = mn0 + ii + q;
-            r[q] = (k < K && i < MN) ? P[i + k * ld] : T(0);
+            r[q] = (FULL || (k < K && i < MN)) ? P[i + k * ld] : T(0);
         }
     } else {
         const int ii = t >> 1;          // 0..127
@@ -74,7 +75,7 @@ __device__ __forceinline__ void load_slab(const T* __restrict__ P, i64 ld, i64 m
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const i64 k = k0 + kk + q;
-            r[q] = (k < K && i < MN) ? P[k + i * ld] : T(0);
+            r[q] = (FULL || (k < K && i < MN)) ? P[k + i * ld] : T(0);
         }
     }
 }
@@ -133,28 +134,28 @@ __device__ __forceinline__ bool tile_of(int bid, int tri, int tiles_m, int tiles
     tn = tri == 1 ? c : r;
     return true;
 }
+// How much of a K-deep update is due once a factorization has recorded `info`: nothing for an
+// update of the failing panel itself (from < 0), else, for an update that gathers the 128-column
+// panels from column `from` on, the panels completed before the failing one.
+__device__ __forceinline__ i64 steps_done(int32_t info, i64 from, i64 K) {
+    if (from < 0 || info < 0) return 0;
+    const i64 f = (i64)info - 1 - from;
+    return f < 0 ? 0 : min(K, f / BM * BM);
+}
 i64 tri_tiles(i64 tiles) {
     const i64 groups = (tiles + 7) / 8;
     return 32 * groups * groups + 4 * groups;
 }
 
-template <typename T, bool TA, bool TB>
-__global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alpha,
-                                                  const T* __restrict__ A, i64 lda,
-                                                  const T* __restrict__ B, i64 ldb, T beta,
-                                                  T* __restrict__ C, i64 ldc, int tri,
-                                                  int tiles_m, int tiles_n,
-                                                  const int32_t* __restrict__ stop) {
+// One 128x128 tile for any operands (FP32, odd leading dimensions, any K): element loads into one LDS
+// slab per operand. FULL: the tile lies inside C and K is a multiple of 16, every load unchecked.
+template <typename T, bool TA, bool TB, bool FULL>
+__device__ __forceinline__ void gemm_tile(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
+                                          const T* __restrict__ B, i64 ldb, T beta, T* __restrict__ C,
+                                          i64 ldc, int tri, i64 m0, i64 n0, T (*As)[BM + PAD],
+                                          T (*Bs)[BN + PAD]) {
     typedef Mfma<T> MF;
     typedef typename MF::acc acc_t;
-    __shared__ T As[BK][BM + PAD];  // As[k][i] = op(A)(m0+i, k0+k)
-    __shared__ T Bs[BK][BN + PAD];  // Bs[k][j] = op(B)(k0+k, n0+j)
-    if (stop && *stop != 0) return;
-
-    int tm, tn;
-    if (!tile_of((int)blockIdx.x, tri, tiles_m, tiles_n, tm, tn)) return;
-    const i64 m0 = (i64)tm * BM, n0 = (i64)tn * BN;
-
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
@@ -165,30 +166,43 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alph
     // read while the first slabs load, and the epilogue is a plain store.
     const bool fold = (beta == T(1)) && (alpha == T(1) || alpha == T(-1));
     const T sgn = fold ? alpha : T(1);
+    // a tile that the triangle does not cut carries no per-entry conditions
+    const bool whole = FULL && fold && (tri == 0 || (tri == 1 ? m0 >= n0 + BN - 1 : n0 >= m0 + BM - 1));
     acc_t acc[4][4];
+    if (whole) {
+        const T* c0 = C + m0 + wm + r16 + (n0 + wn) * ldc;
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) {
-        const i64 m = m0 + wm + mi * 16 + r16;
+        for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni)
+            for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const i64 n = n0 + wn + ni * 16 + MF::row(kq, r);
-                const bool ok = fold && m < M && n < N && !(tri == 1 && m < n) && !(tri == 2 && m > n);
-                acc[mi][ni][r] = ok ? C[m + n * ldc] : T(0);
-            }
+                for (int r = 0; r < 4; ++r)
+                    acc[mi][ni][r] = c0[mi * 16 + (i64)(ni * 16 + MF::row(kq, r)) * ldc];
+    } else {
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi) {
+            const i64 m = m0 + wm + mi * 16 + r16;
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const i64 n = n0 + wn + ni * 16 + MF::row(kq, r);
+                    const bool ok = fold && m < M && n < N && !(tri == 1 && m < n) && !(tri == 2 && m > n);
+                    acc[mi][ni][r] = ok ? C[m + n * ldc] : T(0);
+                }
+        }
     }
 
     T ra[8], rb[8];
-    load_slab<TA>(A, lda, m0, M, 0, K, ra);
-    load_slab<!TB>(B, ldb, n0, N, 0, K, rb);
+    load_slab<TA, FULL>(A, lda, m0, M, 0, K, ra);
+    load_slab<!TB, FULL>(B, ldb, n0, N, 0, K, rb);
     for (i64 k0 = 0; k0 < K; k0 += BK) {
         store_slab<TA>(As, ra, sgn);
         store_slab<!TB>(Bs, rb);
         __syncthreads();
         if (k0 + BK < K) {
-            load_slab<TA>(A, lda, m0, M, k0 + BK, K, ra);
-            load_slab<!TB>(B, ldb, n0, N, k0 + BK, K, rb);
+            load_slab<TA, FULL>(A, lda, m0, M, k0 + BK, K, ra);
+            load_slab<!TB, FULL>(B, ldb, n0, N, k0 + BK, K, rb);
         }
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 4) {
@@ -206,6 +220,17 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alph
         __syncthreads();
     }
 
+    if (whole) {
+        T* c0 = C + m0 + wm + r16 + (n0 + wn) * ldc;
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    c0[mi * 16 + (i64)(ni * 16 + MF::row(kq, r)) * ldc] = acc[mi][ni][r];
+        return;
+    }
     // With the operands fed as (op(B)^T, op(A)^T) the MFMA result is the transpose of the C
     // tile: the lane holds C(m0+wm+mi*16+r16, n0+wn+ni*16+MF::row(kq, r)), r = 0..3.
 #pragma unroll
@@ -226,6 +251,93 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alph
                 else *c = (beta == T(0)) ? alpha * v : __builtin_fma(alpha, v, beta * *c);
             }
         }
+    }
+}
+
+// Both tile kernels: workgroups [0, nfull) take the tiles inside C, in tile_of's order, the others the
+// partial tiles -- one launch, since a second one for a few edge tiles costs a whole tile's latency
+// (28 us at K = 128), but two bodies, since conditions inside one slowed every tile's K loop. full_m,
+// full_n: the grid of whole tiles (0 when K is ragged: then every tile is a checked one).
+struct TileGrid {
+    int nfull, full_m, full_n, tiles_m, tiles_n;
+};
+__device__ __forceinline__ bool pick_tile(const TileGrid& g, int tri, bool& full, i64& m0, i64& n0) {
+    int tm, tn;
+    const int bid = (int)blockIdx.x;
+    full = bid < g.nfull;
+    if (full) {
+        if (!tile_of(bid, tri, g.full_m, g.full_n, tm, tn)) return false;
+    } else {
+        // the partial last tile rows (all, without whole tiles), then the partial last tile column
+        const int q = bid - g.nfull, rows = (g.tiles_m - g.full_m) * g.tiles_n;
+        tm = q < rows ? g.full_m + q / g.tiles_n : q - rows;
+        tn = q < rows ? q % g.tiles_n : g.full_n;
+    }
+    m0 = (i64)tm * BM;
+    n0 = (i64)tn * BN;
+    return !(tri == 1 && n0 > m0 + BM - 1) && !(tri == 2 && m0 > n0 + BN - 1);
+}
+unsigned tile_blocks(i64 m, i64 n, int tri, bool whole, TileGrid& g) {
+    const i64 fm = whole ? m / BM : 0, fn = whole && fm > 0 ? n / BN : 0, ufm = fn > 0 ? fm : 0;
+    const i64 tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
+    const i64 list = ufm > 0 ? ((tri ? tri_tiles(ufm) : ufm * fn) + 7) / 8 * 8 : 0;
+    g = TileGrid{(int)list, (int)ufm, (int)fn, (int)tm, (int)tn};
+    return (unsigned)(list + (tm - ufm) * tn + (fn < tn ? ufm : 0));
+}
+
+template <typename T, bool TA, bool TB>
+__global__ __launch_bounds__(NT, 2) void gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A,
+                                                     i64 lda, const T* __restrict__ B, i64 ldb, T beta,
+                                                     T* __restrict__ C, i64 ldc, int tri, TileGrid g,
+                                                     const int32_t* __restrict__ stop, i64 from) {
+    __shared__ T As[BK][BM + PAD];  // As[k][i] = op(A)(m0+i, k0+k)
+    __shared__ T Bs[BK][BN + PAD];  // Bs[k][j] = op(B)(k0+k, n0+j)
+    if (stop && *stop != 0 && (K = steps_done(*stop, from, K)) <= 0) return;
+    bool full;
+    i64 m0, n0;
+    if (!pick_tile(g, tri, full, m0, n0)) return;
+    if (full) gemm_tile<T, TA, TB, true>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, m0, n0, As, Bs);
+    else gemm_tile<T, TA, TB, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, m0, n0, As, Bs);
+}
+
+// C += sgn A B for at most 16 columns and K <= 128 (the row-echelon form's update of a few
+// right-hand sides): a 16 x 16 tile of C per wave, both operands loaded straight into their lanes,
+// all loads out before the first product. One memory latency and 32 products, 5 us; as 128 x 128
+// tiles with 1 to 16 used columns it took 29 us whatever the height. The products are the FMA chain
+// of the tiled kernels, k ascending.
+constexpr int NARROW = 16, NARROW_K = 128;
+template <typename T>
+__global__ __launch_bounds__(NT) void gemm_narrow_kernel(i64 M, int N, int K, T sgn, const T* __restrict__ A,
+                                                         i64 lda, const T* __restrict__ B, i64 ldb,
+                                                         T* __restrict__ C, i64 ldc,
+                                                         const int32_t* __restrict__ stop) {
+    typedef Mfma<T> MF;
+    if (stop && *stop != 0) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, kq = lane >> 4;
+    const i64 i = (i64)blockIdx.x * 64 + wave * 16 + l16;
+    const bool in = i < M, vin = l16 < N;
+    T a[NARROW_K / 4], b[NARROW_K / 4];
+#pragma unroll
+    for (int kk = 0; kk < NARROW_K / 4; ++kk) {
+        const int k = 4 * kk + kq;
+        a[kk] = (in && k < K) ? A[i + (i64)k * lda] : T(0);
+        b[kk] = (vin && k < K) ? B[k + (i64)l16 * ldb] : T(0);
+    }
+    // D(v, i): lanes run down C's columns
+    typename MF::acc c;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int v = MF::row(kq, r);
+        c[r] = (in && v < N) ? C[i + (i64)v * ldc] : T(0);
+    }
+    const int steps = (K + 3) / 4;
+#pragma unroll
+    for (int kk = 0; kk < NARROW_K / 4; ++kk)
+        if (kk < steps) c = MF::run(b[kk], sgn * a[kk], c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int v = MF::row(kq, r);
+        if (in && v < N) C[i + (i64)v * ldc] = c[r];
     }
 }
 
@@ -417,31 +529,22 @@ __device__ __forceinline__ void dgemm_fast_tile(i64 M, i64 N, i64 K, double alph
 // but with 16-byte operand loads and double-buffered LDS slabs: the next slab is fetched into
 // registers while the current one feeds the MFMAs and is then stored into the other buffer, so
 // each 16-deep step costs one barrier. Edge tiles (partial in m or n) load element by element.
-template <bool TA, bool TB, bool FULL>
+template <bool TA, bool TB>
 __global__ __launch_bounds__(NT, 2) void dgemm_fast_kernel(i64 M, i64 N, i64 K, double alpha,
                                                         const double* __restrict__ A, i64 lda,
                                                         const double* __restrict__ B, i64 ldb,
                                                         double beta, double* __restrict__ C,
-                                                        i64 ldc, int tri, int tiles_m, int tiles_n,
-                                                        const int32_t* __restrict__ stop) {
-    if (stop && *stop != 0) return;
-    int tm, tn;
-    if (FULL) {
-        if (!tile_of((int)blockIdx.x, tri, tiles_m, tiles_n, tm, tn)) return;
-    } else {
-        // the partial last tile row, then the partial last tile column
-        const int fm = (int)(M / BM), fn = (int)(N / BN), row = fm < tiles_m ? tiles_n : 0;
-        const int q = (int)blockIdx.x;
-        tm = q < row ? fm : q - row;
-        tn = q < row ? q : fn;
-    }
-    const i64 m0 = (i64)tm * BM, n0 = (i64)tn * BN;
-    if (tri == 1 && n0 > m0 + BM - 1) return;
-    if (tri == 2 && m0 > n0 + BN - 1) return;
+                                                        i64 ldc, int tri, TileGrid g,
+                                                        const int32_t* __restrict__ stop, i64 from) {
     // As[b][k][i] = sgn op(A)(m0+i, k0+k), Bs[b][k][j] = op(B)(k0+k, n0+j), double-buffered
     __shared__ __align__(16) double As[2][BK][BM + PAD];
     __shared__ __align__(16) double Bs[2][BK][BN + PAD];
-    dgemm_fast_tile<TA, TB, FULL>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, m0, n0, As, Bs);
+    if (stop && *stop != 0 && (K = steps_done(*stop, from, K)) <= 0) return;
+    bool full;
+    i64 m0, n0;
+    if (!pick_tile(g, tri, full, m0, n0)) return;
+    if (full) dgemm_fast_tile<TA, TB, true>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, m0, n0, As, Bs);
+    else dgemm_fast_tile<TA, TB, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, m0, n0, As, Bs);
 }
 
 // The large FP64 products on rocBLAS instead of the hand-written kernels: environment
@@ -479,7 +582,7 @@ __global__ void gate_kernel(const int32_t* __restrict__ stop, double alpha, doub
 template <typename T>
 elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T alpha,
                        const T* A, i64 lda, const T* B, i64 ldb, T beta, T* C, i64 ldc, int tri,
-                       const int32_t* stop, bool allow_library) {
+                       const int32_t* stop, bool allow_library, i64 from = -1) {
     using namespace elx;
     if (m <= 0 || n <= 0) return ELX_SUCCESS;
     ELX_ARG(tri == 0 || m == n);
@@ -492,6 +595,14 @@ elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T a
         return ELX_SUCCESS;
     }
     const double flops = (tri ? 1.0 : 2.0) * (double)m * (double)n * (double)k;
+    if (!ta && !tb && tri == 0 && from < 0 && n <= NARROW && k <= NARROW_K && beta == T(1) &&
+        (alpha == T(1) || alpha == T(-1))) {
+        ProfScope prof_(s, kKDgemm, flops);
+        hipLaunchKernelGGL(gemm_narrow_kernel<T>, dim3((unsigned)((m + 63) / 64)), dim3(NT), 0, s, m, (int)n,
+                           (int)k, alpha, A, lda, B, ldb, C, ldc, stop);
+        ELX_HIP(hipGetLastError());
+        return ELX_SUCCESS;
+    }
     if constexpr (sizeof(T) == 8) {
         // Large FP64 products go to rocBLAS (dgemm, and dsyrk for the symmetric rank-k update:
         // A == B, one operand transposed, one triangle of C) with ELX_DGEMM=library, and so do
@@ -530,53 +641,41 @@ elx_status_t gemm_impl(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, T a
             const double* dB = reinterpret_cast<const double*>(B);
             double* dC = reinterpret_cast<double*>(C);
             const double al = (double)alpha, be = (double)beta;
-            // interior tiles (unchecked), then, if C has partial edge tiles, the checked launch
-            const i64 fm = m / BM, fn = n / BN;
-            const i64 tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
-            ELX_ARG(tm * tn < (i64)1 << 30);
-            auto go = [&](auto full_tag, i64 gm, i64 gn, unsigned blocks) {
-                constexpr bool F = decltype(full_tag)::value;
-                if (gm <= 0 || gn <= 0) return;
-                const int igm = (int)gm, ign = (int)gn;
-                if (!ta && !tb)
-                    hipLaunchKernelGGL((dgemm_fast_kernel<false, false, F>), dim3(blocks), dim3(NT), 0,
-                                       s, m, n, k, al, dA, lda, dB, ldb, be, dC, ldc, tri, igm, ign, stop);
-                else if (!ta && tb)
-                    hipLaunchKernelGGL((dgemm_fast_kernel<false, true, F>), dim3(blocks), dim3(NT), 0,
-                                       s, m, n, k, al, dA, lda, dB, ldb, be, dC, ldc, tri, igm, ign, stop);
-                else if (ta && !tb)
-                    hipLaunchKernelGGL((dgemm_fast_kernel<true, false, F>), dim3(blocks), dim3(NT), 0,
-                                       s, m, n, k, al, dA, lda, dB, ldb, be, dC, ldc, tri, igm, ign, stop);
-                else
-                    hipLaunchKernelGGL((dgemm_fast_kernel<true, true, F>), dim3(blocks), dim3(NT), 0,
-                                       s, m, n, k, al, dA, lda, dB, ldb, be, dC, ldc, tri, igm, ign, stop);
-            };
-            const i64 list = tri ? tri_tiles(fm) : fm * fn;
-            go(std::integral_constant<bool, true>{}, fm, fn, (unsigned)((list + 7) / 8 * 8));
-            const i64 edge = (fm < tm ? tn : 0) + (fn < tn ? fm : 0);
-            if (edge > 0) go(std::integral_constant<bool, false>{}, tm, tn, (unsigned)edge);
+            ELX_ARG(((m + BM - 1) / BM) * ((n + BN - 1) / BN) < (i64)1 << 29);
+            TileGrid g;
+            const dim3 grid(tile_blocks(m, n, tri, true, g));
+            if (!ta && !tb)
+                hipLaunchKernelGGL((dgemm_fast_kernel<false, false>), grid, dim3(NT), 0, s, m, n, k, al, dA, lda,
+                                   dB, ldb, be, dC, ldc, tri, g, stop, from);
+            else if (!ta && tb)
+                hipLaunchKernelGGL((dgemm_fast_kernel<false, true>), grid, dim3(NT), 0, s, m, n, k, al, dA, lda,
+                                   dB, ldb, be, dC, ldc, tri, g, stop, from);
+            else if (ta && !tb)
+                hipLaunchKernelGGL((dgemm_fast_kernel<true, false>), grid, dim3(NT), 0, s, m, n, k, al, dA, lda,
+                                   dB, ldb, be, dC, ldc, tri, g, stop, from);
+            else
+                hipLaunchKernelGGL((dgemm_fast_kernel<true, true>), grid, dim3(NT), 0, s, m, n, k, al, dA, lda,
+                                   dB, ldb, be, dC, ldc, tri, g, stop, from);
             ELX_HIP(hipGetLastError());
             return ELX_SUCCESS;
         }
     }
-    const i64 tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
-    ELX_ARG(tm * tn < (i64)1 << 30);
+    ELX_ARG(((m + BM - 1) / BM) * ((n + BN - 1) / BN) < (i64)1 << 29);
     ProfScope prof_(s, kKDgemm, flops);
-    const i64 list = tri ? tri_tiles(tm) : tm * tn;
-    const unsigned blocks = (unsigned)((list + 7) / 8 * 8);
-    const int itm = (int)tm, itn = (int)tn;
+    TileGrid g;
+    const dim3 grid(tile_blocks(m, n, tri, k % BK == 0, g));
     if (!ta && !tb)
-        hipLaunchKernelGGL((gemm_kernel<T, false, false>), dim3(blocks), dim3(NT), 0, s, m, n, k,
-                           alpha, A, lda, B, ldb, beta, C, ldc, tri, itm, itn, stop);
+        hipLaunchKernelGGL((gemm_kernel<T, false, false>), grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, B, ldb,
+                           beta, C, ldc, tri, g, stop, from);
     else if (!ta && tb)
-        hipLaunchKernelGGL((gemm_kernel<T, false, true>), dim3(blocks), dim3(NT), 0, s, m, n, k,
-                           alpha, A, lda, B, ldb, beta, C, ldc, tri, itm, itn, stop);
+        hipLaunchKernelGGL((gemm_kernel<T, false, true>), grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, B, ldb,
+                           beta, C, ldc, tri, g, stop, from);
     else if (ta && !tb)
-        hipLaunchKernelGGL((gemm_kernel<T, true, false>), dim3(blocks), dim3(NT), 0, s, m, n, k,
-                           alpha, A, lda, B, ldb, beta, C, ldc, tri, itm, itn, stop);
+        hipLaunchKernelGGL((gemm_kernel<T, true, false>), grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, B, ldb,
+                           beta, C, ldc, tri, g, stop, from);
     else
-        hipLaunchKernelGGL((gemm_kernel<T, true, true>), dim3(blocks), dim3(NT), 0, s, m, n, k,
-                           alpha, A, lda, B, ldb, beta, C, ldc, tri, itm, itn, stop);
+        hipLaunchKernelGGL((gemm_kernel<T, true, true>), grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, B, ldb,
+                           beta, C, ldc, tri, g, stop, from);
     ELX_HIP(hipGetLastError());
     return ELX_SUCCESS;
 }
@@ -597,6 +696,21 @@ elx_status_t launch_gemm(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, f
                          i64 ldc, int tri, const int32_t* stop, bool allow_library) {
     return gemm_impl<float>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri, stop,
                             allow_library);
+}
+
+bool gemm_library_selected() { return !dgemm_own_selected(); }
+
+elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, double alpha,
+                              const double* A, i64 lda, const double* B, i64 ldb, double beta,
+                              double* C, i64 ldc, int tri, const int32_t* stop, i64 from) {
+    return gemm_impl<double>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri, stop, false,
+                             from);
+}
+elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, float alpha,
+                              const float* A, i64 lda, const float* B, i64 ldb, float beta, float* C,
+                              i64 ldc, int tri, const int32_t* stop, i64 from) {
+    return gemm_impl<float>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri, stop, false,
+                            from);
 }
 
 elx_status_t launch_dgemm(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, double alpha,
