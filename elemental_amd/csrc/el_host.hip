@@ -188,6 +188,17 @@ struct DevBuf {
     DevBuf& operator=(const DevBuf&) = delete;
 };
 
+// A column-major matrix of m x n elements between leading dimensions. Where both sides are
+// contiguous it is one linear copy: the runtime takes a 2-D copy of pageable memory row by row
+// through its staging buffer.
+void copy_matrix(void* dst, size_t ldd, const void* src, size_t lds, size_t m, size_t n, size_t size,
+                 hipMemcpyKind kind) {
+    if ((ldd == m && lds == m) || n == 1)
+        hcheck(hipMemcpy(dst, src, size * m * n, kind), "hipMemcpy");
+    else
+        hcheck(hipMemcpy2D(dst, size * ldd, src, size * lds, size * m, n, kind), "hipMemcpy2D");
+}
+
 // Device copy of a host matrix with leading dimension max(height,1).
 template <typename T>
 struct DevMatrix {
@@ -198,16 +209,14 @@ struct DevMatrix {
         : m(A.Height()), n(A.Width()), ld(std::max(A.Height(), 1)),
           buf(sizeof(T) * (size_t)ld * (size_t)A.Width()) {
         if (m > 0 && n > 0)
-            hcheck(hipMemcpy2D(buf.p, sizeof(T) * ld, A.LockedBuffer(), sizeof(T) * A.LDim(),
-                               sizeof(T) * m, n, hipMemcpyHostToDevice),
-                   "hipMemcpy2D");
+            copy_matrix(buf.p, (size_t)ld, A.LockedBuffer(), (size_t)A.LDim(), (size_t)m, (size_t)n, sizeof(T),
+                        hipMemcpyHostToDevice);
     }
     T* ptr() { return static_cast<T*>(buf.p); }
     void to_host(Matrix<T>& A) {
         if (m > 0 && n > 0)
-            hcheck(hipMemcpy2D(A.Buffer(), sizeof(T) * A.LDim(), buf.p, sizeof(T) * ld,
-                               sizeof(T) * m, n, hipMemcpyDeviceToHost),
-                   "hipMemcpy2D");
+            copy_matrix(A.Buffer(), (size_t)A.LDim(), buf.p, (size_t)ld, (size_t)m, (size_t)n, sizeof(T),
+                        hipMemcpyDeviceToHost);
     }
 };
 
