@@ -30,6 +30,7 @@
 
 #include "batched_tuning.hpp"
 #include "elx_common.hpp"
+#include "wave.hpp"
 
 namespace {
 
@@ -94,14 +95,7 @@ __device__ __forceinline__ float bcast(float v, int src) {
 template <typename T>
 using gmem = __attribute__((address_space(1))) T;
 
-// Compile-time loop: f(std::integral_constant<int, i>) for i = B .. E-1.
-template <int B, int E, typename Fn>
-__device__ __forceinline__ void static_for(Fn&& f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
+using elx::wv::static_for;
 
 // S[kk * SM + r] = A(k0 + r, c0 + kk) for r < m, kk < kc, zero for kc <= kk < kcp: threads
 // walk the (row, column) pairs column by column (coalesced), 16 loads in flight per thread.
@@ -956,146 +950,209 @@ __global__ __launch_bounds__(BNT, kWideOcc) void potrf_wide_vbatched_kernel(
     }
 }
 
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
 // One workgroup: L L^T X = B for one matrix (L from potrf), up to NR right-hand sides at a time
-// in LDS, blocked by SB = 32 rows. Forward (right-looking): wave 0 solves the diagonal block
-// with its rows in registers, then every row below subtracts the block's products (a row per
-// thread). Backward: each block column's dot products with the solved part below (a wave per
-// column, lanes down the column), then wave 0 solves the transposed diagonal block with its
-// columns in registers.
-constexpr int NR = 8, SB = 32, SLD = SB + 1;
+// in LDS, blocked by SB = 32 rows. Forward (right-looking): wave 0 solves the diagonal block,
+// then every row below subtracts the block's products, 16 rows x 8 columns per wave on the matrix
+// cores. Backward: the block column's products with the solved part below on the matrix cores,
+// the waves splitting its rows, then wave 0 solves the transposed diagonal block.
+// The diagonal solves hold a row per lane of a 16-lane group and two columns per group, the 32
+// rows in two halves: a step's solved entry reaches its group by one DPP broadcast per column,
+// against two readlanes, a masked product and a masked FMA for each of the 8 columns when a lane
+// held a row of all of them; a row per thread read 8 entries of Y from LDS per factor entry, and
+// a wave per column of the backward products spent 48 shuffles on its sums.
+constexpr int NR = 8, SB = 32, SLD = SB + 1, YLD = BNMAX + 2, PW = BNT / 64;
 template <typename T>
 __device__ __forceinline__ void potrs_one(int n, const gmem<T>* L, int lda, gmem<T>* B, int ldb,
                                           int nrhs, T* Y, T* Part, T* Lb) {
+    typedef elx::wv::Mfma4<T> MF;
+    using elx::wv::row_bcast;
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int l16 = lane & 15, kq = lane >> 4;
     const int nblk = (n + SB - 1) / SB;
     auto stage_l11 = [&](int k0, int kb) {
-        for (int idx = t; idx < kb * kb; idx += BNT) {
-            const int i = idx % kb, j = idx / kb;
-            Lb[i * SLD + j] = (i >= j) ? L[(k0 + i) + (size_t)(k0 + j) * lda] : T(0);
+        for (int idx = t; idx < SB * SB; idx += BNT) {
+            const int i = idx % SB, j = idx / SB;
+            Lb[i * SLD + j] = (i >= j && i < kb) ? L[(k0 + i) + (size_t)(k0 + j) * lda] : T(0);
         }
     };
     for (int c0 = 0; c0 < nrhs; c0 += NR) {
         const int nr = min(NR, nrhs - c0);
         for (int idx = t; idx < n * nr; idx += BNT) {
             const int i = idx % n, c = idx / n;
-            Y[c * BNMAX + i] = B[i + (size_t)(c0 + c) * ldb];
+            Y[c * YLD + i] = B[i + (size_t)(c0 + c) * ldb];
         }
         __syncthreads();
-        // forward: L y = b (dtrsm Left Lower NoTrans NonUnit), right-looking by 32-row blocks:
-        // the diagonal block's solve, then its products subtracted from every row below (a
-        // row per thread: the block's 32 columns of L are independent loads, coalesced across
-        // the threads)
+        // forward: L y = b (dtrsm Left Lower NoTrans NonUnit), right-looking by 32-row blocks
         for (int b = 0; b < nblk; ++b) {
-            const int k0 = b * SB, kb = min(SB, n - k0);
+            const int k0 = b * SB, kb = min(SB, n - k0), r0 = k0 + kb;
             stage_l11(k0, kb);
             __syncthreads();
             if (wave == 0) {
-                T lrow[SB], yv[NR];
+                // rows l16 and 16 + l16 of columns 2 kq and 2 kq + 1
+                T la[16], lb[16], lc[16], y0[2], y1[2];
 #pragma unroll
-                for (int j = 0; j < SB; ++j) lrow[j] = (lane < kb) ? Lb[lane * SLD + j] : T(0);
-#pragma unroll
-                for (int q = 0; q < NR; ++q) yv[q] = (lane < kb && q < nr) ? Y[q * BNMAX + k0 + lane] : T(0);
-                // reciprocals of the diagonal, one division per lane, broadcast per step
-                const T dinv = (lane < kb) ? T(1) / Lb[lane * SLD + lane] : T(0);
-#pragma unroll
-                for (int k = 0; k < SB; ++k) {
-                    if (k < kb) {
-                        const T dk = bcast(dinv, k);
-                        // every column slot, branch-free (slots >= nr hold zeros): a guard per
-                        // slot would split the step chain into small branch blocks
-#pragma unroll
-                        for (int q = 0; q < NR; ++q) {
-                            if (lane == k) yv[q] = yv[q] * dk;
-                            const T yk = bcast(yv[q], k);
-                            if (lane > k) yv[q] = __builtin_fma(-lrow[k], yk, yv[q]);
-                        }
-                    }
+                for (int k = 0; k < 16; ++k) {
+                    la[k] = Lb[l16 * SLD + k];
+                    lb[k] = Lb[(16 + l16) * SLD + k];
+                    lc[k] = Lb[(16 + l16) * SLD + 16 + k];
                 }
-                if (lane < kb)
+                const T d0 = (l16 < kb) ? T(1) / Lb[l16 * SLD + l16] : T(0);
+                const T d1 = (16 + l16 < kb) ? T(1) / Lb[(16 + l16) * SLD + 16 + l16] : T(0);
 #pragma unroll
-                    for (int q = 0; q < NR; ++q)
-                        if (q < nr) Y[q * BNMAX + k0 + lane] = yv[q];
+                for (int s = 0; s < 2; ++s) {
+                    const int q = 2 * kq + s;
+                    y0[s] = (l16 < kb && q < nr) ? Y[q * YLD + k0 + l16] : T(0);
+                    y1[s] = (16 + l16 < kb && q < nr) ? Y[q * YLD + k0 + 16 + l16] : T(0);
+                }
+                static_for<0, 16>([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    const T dk = row_bcast<k>(d0);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        const T yk = row_bcast<k>(y0[s]) * dk;
+                        y0[s] = l16 == k ? yk : (l16 > k ? __builtin_fma(-la[k], yk, y0[s]) : y0[s]);
+                        y1[s] = __builtin_fma(-lb[k], yk, y1[s]);
+                    }
+                });
+                static_for<0, 16>([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    const T dk = row_bcast<k>(d1);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        const T yk = row_bcast<k>(y1[s]) * dk;
+                        y1[s] = l16 == k ? yk : (l16 > k ? __builtin_fma(-lc[k], yk, y1[s]) : y1[s]);
+                    }
+                });
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int q = 2 * kq + s;
+                    if (q < nr && l16 < kb) Y[q * YLD + k0 + l16] = y0[s];
+                    if (q < nr && 16 + l16 < kb) Y[q * YLD + k0 + 16 + l16] = y1[s];
+                }
             }
             __syncthreads();
-            for (int i = k0 + kb + t; i < n; i += BNT) {
-                T acc[NR];
+            if (r0 < n) {  // a full block: kb == SB
+                T yo[SB / 4];
 #pragma unroll
-                for (int q = 0; q < NR; ++q) acc[q] = (q < nr) ? Y[q * BNMAX + i] : T(0);
-                const gmem<T>* li = L + i + (size_t)k0 * lda;
-#pragma unroll 8
-                for (int k = 0; k < kb; ++k) {
-                    const T l = li[(size_t)k * lda];
+                for (int kk = 0; kk < SB / 4; ++kk)
+                    yo[kk] = l16 < nr ? -Y[l16 * YLD + k0 + 4 * kk + kq] : T(0);
+                for (int i0 = r0 + 16 * wave; i0 < n; i0 += 16 * PW) {
+                    const int i = i0 + l16;
+                    const bool in = i < n;
+                    const gmem<T>* li = L + (in ? i : 0) + (size_t)(k0 + kq) * lda;
+                    T lo[SB / 4];
 #pragma unroll
-                    for (int q = 0; q < NR; ++q)
-                        if (q < nr) acc[q] = __builtin_fma(-l, Y[q * BNMAX + k0 + k], acc[q]);
+                    for (int kk = 0; kk < SB / 4; ++kk) lo[kk] = in ? li[(size_t)(4 * kk) * lda] : T(0);
+                    typename MF::acc acc;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int q = MF::row(kq, r);
+                        acc[r] = (in && q < nr) ? Y[q * YLD + i] : T(0);
+                    }
+#pragma unroll
+                    for (int kk = 0; kk < SB / 4; ++kk) acc = MF::run(yo[kk], lo[kk], acc);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int q = MF::row(kq, r);
+                        if (in && q < nr) Y[q * YLD + i] = acc[r];
+                    }
                 }
-#pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    if (q < nr) Y[q * BNMAX + i] = acc[q];
             }
             __syncthreads();
         }
         // backward: L^T x = y (dtrsm Left Lower Trans NonUnit), blocks from the bottom
         for (int b = nblk - 1; b >= 0; --b) {
             const int k0 = b * SB, kb = min(SB, n - k0), r0 = k0 + kb;
-            for (int j = wave; j < kb; j += 4) {
-                T acc[NR];
+            if (r0 < n) {
+                // P(q, j) = sum over the rows below of L(i, j) x(i, q): 16 rows per wave and turn
+                typename MF::acc acc[2];
 #pragma unroll
-                for (int q = 0; q < NR; ++q) acc[q] = T(0);
-                const gmem<T>* col = L + (size_t)(k0 + j) * lda;
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[j][r] = T(0);
+                const gmem<T>* c = L + (size_t)(k0 + l16) * lda;
 #pragma unroll 2
-                for (int i = r0 + lane; i < n; i += 64) {
-                    const T l = col[i];
+                for (int i0 = r0 + 16 * wave; i0 < n; i0 += 16 * PW) {
+                    T xo[4], l0[4], l1[4];
 #pragma unroll
-                    for (int q = 0; q < NR; ++q)
-                        if (q < nr) acc[q] = __builtin_fma(l, Y[q * BNMAX + i], acc[q]);
+                    for (int kk = 0; kk < 4; ++kk) {
+                        const int i = i0 + 4 * kk + kq;
+                        const bool in = i < n;
+                        l0[kk] = in ? c[i] : T(0);
+                        l1[kk] = in ? c[i + (size_t)16 * lda] : T(0);
+                        xo[kk] = (in && l16 < nr) ? Y[l16 * YLD + i] : T(0);
+                    }
+#pragma unroll
+                    for (int kk = 0; kk < 4; ++kk) {
+                        acc[0] = MF::run(xo[kk], l0[kk], acc[0]);
+                        acc[1] = MF::run(xo[kk], l1[kk], acc[1]);
+                    }
                 }
 #pragma unroll
-                for (int q = 0; q < NR; ++q) acc[q] = wave_sum(acc[q]);
-                if (lane == 0)
+                for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int q = 0; q < NR; ++q) Part[j * NR + q] = acc[q];
+                    for (int r = 0; r < 4; ++r) {
+                        const int q = MF::row(kq, r);
+                        if (q < NR) Part[(wave * NR + q) * SB + 16 * j + l16] = acc[j][r];
+                    }
             }
             stage_l11(k0, kb);
             __syncthreads();
             if (wave == 0) {
-                // lane k holds column k of L11: L(i, k) for every i
-                T lcol[SB], xv[NR];
+                // columns l16 and 16 + l16 of L11: L(i, .) for the rows i below
+                T la[16], lb[16], lc[16], x0[2], x1[2];
 #pragma unroll
-                for (int i = 0; i < SB; ++i) lcol[i] = (lane < kb) ? Lb[i * SLD + lane] : T(0);
-#pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    xv[q] = (lane < kb && q < nr) ? Y[q * BNMAX + k0 + lane] - Part[lane * NR + q] : T(0);
-                const T dinv = (lane < kb) ? T(1) / Lb[lane * SLD + lane] : T(0);
-#pragma unroll
-                for (int i = SB - 1; i >= 0; --i) {
-                    if (i < kb) {
-                        const T di = bcast(dinv, i);
-#pragma unroll
-                        for (int q = 0; q < NR; ++q) {
-                            if (lane == i) xv[q] = xv[q] * di;
-                            const T xi = bcast(xv[q], i);
-                            if (lane < i) xv[q] = __builtin_fma(-lcol[i], xi, xv[q]);
-                        }
-                    }
+                for (int i = 0; i < 16; ++i) {
+                    la[i] = Lb[i * SLD + l16];
+                    lb[i] = Lb[(16 + i) * SLD + l16];
+                    lc[i] = Lb[(16 + i) * SLD + 16 + l16];
                 }
-                if (lane < kb)
+                const T d0 = (l16 < kb) ? T(1) / Lb[l16 * SLD + l16] : T(0);
+                const T d1 = (16 + l16 < kb) ? T(1) / Lb[(16 + l16) * SLD + 16 + l16] : T(0);
 #pragma unroll
-                    for (int q = 0; q < NR; ++q)
-                        if (q < nr) Y[q * BNMAX + k0 + lane] = xv[q];
+                for (int s = 0; s < 2; ++s) {
+                    const int q = 2 * kq + s;
+                    T p0 = T(0), p1 = T(0);
+                    if (r0 < n)
+#pragma unroll
+                        for (int w = 0; w < PW; ++w) {
+                            p0 += Part[(w * NR + q) * SB + l16];
+                            p1 += Part[(w * NR + q) * SB + 16 + l16];
+                        }
+                    x0[s] = (l16 < kb && q < nr) ? Y[q * YLD + k0 + l16] - p0 : T(0);
+                    x1[s] = (16 + l16 < kb && q < nr) ? Y[q * YLD + k0 + 16 + l16] - p1 : T(0);
+                }
+                static_for<0, 16>([&](auto ic) {
+                    constexpr int i = 15 - decltype(ic)::value;
+                    const T di = row_bcast<i>(d1);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        const T xi = row_bcast<i>(x1[s]) * di;
+                        x1[s] = l16 == i ? xi : (l16 < i ? __builtin_fma(-lc[i], xi, x1[s]) : x1[s]);
+                        x0[s] = __builtin_fma(-lb[i], xi, x0[s]);
+                    }
+                });
+                static_for<0, 16>([&](auto ic) {
+                    constexpr int i = 15 - decltype(ic)::value;
+                    const T di = row_bcast<i>(d0);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        const T xi = row_bcast<i>(x0[s]) * di;
+                        x0[s] = l16 == i ? xi : (l16 < i ? __builtin_fma(-la[i], xi, x0[s]) : x0[s]);
+                    }
+                });
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int q = 2 * kq + s;
+                    if (q < nr && l16 < kb) Y[q * YLD + k0 + l16] = x0[s];
+                    if (q < nr && 16 + l16 < kb) Y[q * YLD + k0 + 16 + l16] = x1[s];
+                }
             }
             __syncthreads();
         }
         for (int idx = t; idx < n * nr; idx += BNT) {
             const int i = idx % n, c = idx / n;
-            B[i + (size_t)(c0 + c) * ldb] = Y[c * BNMAX + i];
+            B[i + (size_t)(c0 + c) * ldb] = Y[c * YLD + i];
         }
         __syncthreads();
     }
@@ -1106,8 +1163,8 @@ template <typename T>
 __global__ __launch_bounds__(BNT, 2) void potrs_vbatched_kernel(
     const BatchItem* __restrict__ items, int count, const T* const* __restrict__ Ls,
     T* const* __restrict__ Bs, const int32_t* __restrict__ info, int* queue) {
-    __shared__ T Y[NR * BNMAX];
-    __shared__ T Part[SB * NR];
+    __shared__ T Y[NR * YLD];
+    __shared__ T Part[PW * SB * NR];
     __shared__ T Lb[SB * SLD];
     __shared__ int s_i;
     for (;;) {
