@@ -135,7 +135,7 @@ CLASS_KERNELS = {
                   "void (anonymous namespace)::lu_panel_kernel<float>"), ()),
     "lpgemm": (("void (anonymous namespace)::lpgemm_kernel",), ()),
     "row_moves": (("(anonymous namespace)::row_moves_rowmajor_kernel",), ()),
-    "trsm_small": (("void (anonymous namespace)::trsm_small_kernel<float>",
+    "trsm_small": (("void (anonymous namespace)::trsm_block_kernel<float",
                     "(anonymous namespace)::trmm_inv_kernel"), ()),
     "trsv": (("(anonymous namespace)::trsv_kernel",), ()),
     "residual_f64": (("(anonymous namespace)::gemv_partial_kernel",),

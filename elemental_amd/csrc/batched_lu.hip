@@ -14,7 +14,7 @@
 //      accumulation) with the U operand scaled by a power of two below 2^15.
 //   3. Refinement in FP64: x = M^-1 b, then r = b - A x with A read in FP64; plain IR while a
 //      step cuts the backward error at least 3x (a candidate kept only when the residual
-//      decreased, Refined.hpp:96-105), then right-preconditioned FGMRES(30) (modified
+//      decreased, Refined.hpp:96-105), then right-preconditioned FGMRES(30) (classical
 //      Gram-Schmidt applied twice, Givens rotations), until ||r||inf / (||A||inf ||x||inf +
 //      ||b||inf) <= tol.
 //   4. A system whose refinement stalls (or whose low-precision factorization meets an exactly

@@ -125,7 +125,7 @@ elx_status_t scratch_get(int slot, size_t bytes, void** out) {
     return ELX_SUCCESS;
 }
 
-// The exchange area of the cooperative panel kernel is uncached device memory (coherent
+// The exchange area of the LDS panel kernel is uncached device memory (coherent
 // across XCDs without cache maintenance). Uncached memory that a kernel has read is never
 // freed before the process ends; a larger area replaces a smaller one and the old one is
 // kept.

@@ -68,7 +68,7 @@ constexpr int kSlotFullPiv = 65;
 // scratch slot of the register panel's move list and row origins
 constexpr int kSlotRPanel = 66;
 
-// Per-device persistent state of the cooperative panel kernel's exchange area.
+// Per-device persistent state of the LDS panel kernel's exchange area.
 struct PanelSync {
     int64_t* flags = nullptr;  // one per workgroup, monotonically increasing
     void* slots = nullptr;     // candidate exchange area

@@ -1,4 +1,5 @@
-// Partial-pivoting LU panel as one cooperative, LDS-resident kernel.
+// Partial-pivoting LU panel as one LDS-resident kernel over up to 256 workgroups, for the panels
+// that the register-resident panel (lu_rpanel.hip) does not take; launch_panel below says which.
 //
 // Restates lu::Panel (src/lapack_like/factor/LU/Panel.hpp:15-60): for every column c of the
 // mp x w panel, take the first row of largest |a(i,c)| among rows c..mp-1 (blas::MaxInd =

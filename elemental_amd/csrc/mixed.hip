@@ -179,7 +179,7 @@ elx_status_t lp_update(Ctx& c, i64 m, i64 n, i64 k, const float* Lt, const float
 }
 
 // Two-level blocked LU with partial pivoting of W (fp32, A stored row by row, so a row
-// interchange moves contiguous memory): cooperative panels inside NB-column outer blocks; the
+// interchange moves contiguous memory): multi-workgroup panels inside NB-column outer blocks; the
 // outer trailing update is one rank-NB low-precision GEMM. Panels are 32 columns wide and run
 // on the CUs of one XCD, exchanging their pivot candidates through its L2, when the rows fit
 // there (up to 1024 per CU), else 128 columns over all XCDs through memory.
@@ -471,7 +471,7 @@ static elx_status_t mixed_solve(int kind, void* stream, int64_t n, int64_t nrhs,
     ELX_CHECK(d2h(&finfo, c.info, 1, s));
     ELX_CHECK(d2h(&anorm, anorm_d, 1, s));
     st.factor_info = finfo;
-    // the cooperative panel gave up waiting for a peer workgroup: a device error, not a
+    // the panel gave up waiting for a peer workgroup: a device error, not a
     // numerical outcome
     if (finfo < 0) {
         if (stats) *stats = st;

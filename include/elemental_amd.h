@@ -15,9 +15,10 @@
  *                    SingularMatrixException / NonHPDMatrixException. The rest of the
  *                    enqueued sequence then changes nothing, so A (and B) are left as the
  *                    reference leaves them when it throws.
- *   *dInfo == -1     the cooperative LU panel gave up waiting for a peer workgroup (a GPU
- *                    shared with other work can delay one); A is unchanged from the start of
- *                    that panel (its current 32-column block) on. A runtime error, not a numerical result.
+ *   *dInfo == -1     the LU panel gave up waiting for a peer workgroup (a GPU shared with
+ *                    other work can delay one); A is unchanged from the start of that panel
+ *                    (its current 32-column block) on. A runtime error, not a numerical
+ *                    result.
  * Block sizes nb > 128 run as 128-column panels (the same pivots in exact arithmetic).
  *
  * Every routine of the plain path exists for FP64 (elx_d*) and FP32 (elx_s*), as the
