@@ -190,27 +190,39 @@ elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out) {
     return ELX_SUCCESS;
 }
 
-elx_status_t chain_sync_get(size_t bytes, ChainSync** out) {
+bool chain_sync_get(size_t bytes, bool capturing, ChainSync** out) {
     int dev = 0;
-    ELX_HIP(hipGetDevice(&dev));
+    if (hipGetDevice(&dev) != hipSuccess) return false;
     std::lock_guard<std::mutex> lk(g_mu);
     ChainSync& cs = g_csync[dev];
+    *out = &cs;
+    if (cs.ctrl && cs.bytes >= bytes) return true;
+    if (capturing) return false;
+    auto failed = [](hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e != hipSuccess;
+    };
+    if (!cs.last && failed(hipEventCreateWithFlags(&cs.last, hipEventDisableTiming))) return false;
     if (!cs.ctrl) {
         const uint32_t first[2] = {1u, 0u};  // epoch, workgroups finished
-        ELX_HIP(hipMalloc(&cs.ctrl, sizeof(first)));
-        ELX_HIP(hipMemcpy(cs.ctrl, first, sizeof(first), hipMemcpyHostToDevice));
+        void* ctrl = nullptr;
+        if (failed(hipMalloc(&ctrl, sizeof(first)))) return false;
+        if (failed(hipMemcpy(ctrl, first, sizeof(first), hipMemcpyHostToDevice))) {
+            (void)hipFree(ctrl);
+            return false;
+        }
+        cs.ctrl = ctrl;
     }
     if (cs.bytes < bytes) {
         // the smaller area stays: queued launches may still use it, and uncached memory that a
         // kernel has read is not freed
         const size_t want = std::max<size_t>(std::max<size_t>(bytes, 2 * cs.bytes), (size_t)4 << 20);
         void* area = nullptr;
-        ELX_HIP(hipExtMallocWithFlags(&area, want, hipDeviceMallocUncached));
+        if (failed(hipExtMallocWithFlags(&area, want, hipDeviceMallocUncached))) return false;
         cs.area = area;
         cs.bytes = want;
     }
-    *out = &cs;
-    return ELX_SUCCESS;
+    return true;
 }
 
 // ---------------------------------------------------------------- kernel-class timing
@@ -338,8 +350,11 @@ elx_status_t trsm_blocked(hipStream_t s, int side, int uplo, int orient, int dia
     const i64 bs = 128;
     // few right-hand sides: one chained launch instead of a diagonal solve and a GEMM per block
     // (not where nothing may be allocated: its hand-off area is)
-    if (side == kLeft && allow_library && n <= kChainRhs && !(dot_order && m <= bs))
-        return launch_solve_chain(s, uplo, orient, diag, m, n, A, lda, B, ldb, stop);
+    if (side == kLeft && allow_library && n <= kChainRhs && !(dot_order && m <= bs)) {
+        bool taken = false;
+        ELX_CHECK(launch_solve_chain(s, uplo, orient, diag, m, n, A, lda, B, ldb, stop, &taken));
+        if (taken) return ELX_SUCCESS;
+    }
     if (side == kLeft) {
         if (m <= bs)
             return launch_trsm_small(s, side, uplo, orient, diag, m, n, A, lda, B, ldb, stop, dot_order);

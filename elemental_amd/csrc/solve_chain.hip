@@ -21,10 +21,13 @@
 // The hand-off is through uncached memory in tagged 16-byte units (exchange.hpp): a unit holds
 // eight bytes of the solution, the launch's epoch and a hash, so a reader needs no flag or store
 // completion. The epoch lives in device memory and the last workgroup advances it, so replays of
-// a captured launch never take an earlier replay's units for their own. Each block waits only on
+// a captured launch never take an earlier replay's units for their own. The area is one per
+// device, so launches from several streams wait for each other; where it cannot be had (a capture
+// that would have to allocate it, no memory left) the caller's blocked sequence runs instead. Each block waits only on
 // earlier blocks, which resident workgroups own; every wait is bounded, and a wait that runs out
 // turns the solution into NaN instead of hanging.
 #include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 #include "elx_common.hpp"
@@ -331,15 +334,24 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
 
 template <typename T>
 elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs, const T* A, i64 lda,
-                        T* B, i64 ldb, const int32_t* stop) {
+                        T* B, i64 ldb, const int32_t* stop, bool* taken) {
     const elx::DeviceInfo& di = elx::device_info();
     const i64 nblk = (n + BS - 1) / BS;
-    elx::ProfScope prof_(s, elx::kKTrsm, (double)n * (double)n * (double)nrhs);
     const size_t units = (size_t)nblk * (BS * NV / Unit<T>::PER);
     const i64 most = std::min<i64>(MAX_GROUPS, (nrhs + NV - 1) / NV);
     ELX_ARG(units < ((size_t)1 << 27));
+    *taken = false;
+    // a capture can neither allocate nor wait for an event from outside it; a status that cannot
+    // be had (another stream's capture forbids the call) counts as one
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    const hipError_t se = hipStreamIsCapturing(s, &st);
+    if (se != hipSuccess) (void)hipGetLastError();
+    const bool capturing = se != hipSuccess || st != hipStreamCaptureStatusNone;
     elx::ChainSync* sync = nullptr;
-    ELX_CHECK(elx::chain_sync_get(units * sizeof(u4) * (size_t)most, &sync));
+    if (!elx::chain_sync_get(units * sizeof(u4) * (size_t)most, capturing, &sync)) return ELX_SUCCESS;
+    std::lock_guard<std::mutex> lk(sync->mu);
+    if (!capturing && sync->recorded && sync->stream != s) ELX_HIP(hipStreamWaitEvent(s, sync->last, 0));
+    elx::ProfScope prof_(s, elx::kKTrsm, (double)n * (double)n * (double)nrhs);
     ChainArgs<T> a;
     a.n = n;
     a.A = A;
@@ -372,6 +384,12 @@ elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i6
         else ELX_CHECK(diag == elx::kUnit ? go(yes, four) : go(no, four));
         ELX_HIP(hipGetLastError());
     }
+    if (!capturing) {
+        ELX_HIP(hipEventRecord(sync->last, s));
+        sync->stream = s;
+        sync->recorded = true;
+    }
+    *taken = true;
     return ELX_SUCCESS;
 }
 
@@ -380,12 +398,14 @@ elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i6
 namespace elx {
 
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
-                                const double* A, i64 lda, double* B, i64 ldb, const int32_t* stop) {
-    return chain_impl<double>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, stop);
+                                const double* A, i64 lda, double* B, i64 ldb, const int32_t* stop,
+                                bool* taken) {
+    return chain_impl<double>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, stop, taken);
 }
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
-                                const float* A, i64 lda, float* B, i64 ldb, const int32_t* stop) {
-    return chain_impl<float>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, stop);
+                                const float* A, i64 lda, float* B, i64 ldb, const int32_t* stop,
+                                bool* taken) {
+    return chain_impl<float>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, stop, taken);
 }
 
 }  // namespace elx

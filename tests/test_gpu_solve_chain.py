@@ -73,3 +73,43 @@ def test_captured_solves_replay(dev):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(dB, eager)
+
+
+def test_capture_that_would_have_to_allocate(dev):
+    """A first solve of its size, under capture: it runs without the hand-off area's growth and
+    replays to the eager result bit for bit."""
+    n, r = 4400, 128
+    rng = np.random.default_rng(3)
+    dT = dev.to_device(np.tril(rng.standard_normal((n, n)) / n) + np.eye(n))
+    B = torch.from_numpy(rng.standard_normal((n, r)))
+    dB = dev.to_device(np.zeros((n, r)))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        dev.trsm(0, 0, 0, 0, 1.0, dT, dB)
+    for _ in range(3):
+        dB.copy_(B)
+        g.replay()
+        eager = dev.to_device(B.numpy())
+        torch.cuda.synchronize()
+        dev.trsm(0, 0, 0, 0, 1.0, dT, eager)
+        torch.cuda.synchronize()
+        assert torch.equal(dB, eager)
+
+
+def test_two_streams(dev):
+    """Solves queued on two streams without any wait between them."""
+    n = 1500
+    rng = np.random.default_rng(4)
+    dT = dev.to_device(np.tril(rng.standard_normal((n, n)) / n) + np.eye(n))
+    B = rng.standard_normal((n, 2))
+    want = dev.to_device(B)
+    dev.trsm(0, 0, 0, 0, 1.0, dT, want)
+    got = [dev.to_device(B) for _ in range(16)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for q, dB in enumerate(got):
+        with torch.cuda.stream(streams[q % 2]):
+            dev.trsm(0, 0, 0, 0, 1.0, dT, dB)
+    torch.cuda.synchronize()
+    for dB in got:
+        assert torch.equal(dB, want)
