@@ -190,39 +190,47 @@ elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out) {
     return ELX_SUCCESS;
 }
 
-bool chain_sync_get(size_t bytes, bool capturing, ChainSync** out) {
+elx_status_t chain_sync_get(ChainSync** out) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
+    ELX_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_mu);
-    ChainSync& cs = g_csync[dev];
-    *out = &cs;
-    if (cs.ctrl && cs.bytes >= bytes) return true;
-    if (capturing) return false;
-    auto failed = [](hipError_t e) {
-        if (e != hipSuccess) (void)hipGetLastError();
-        return e != hipSuccess;
-    };
-    if (!cs.last && failed(hipEventCreateWithFlags(&cs.last, hipEventDisableTiming))) return false;
-    if (!cs.ctrl) {
-        const uint32_t first[2] = {1u, 0u};  // epoch, workgroups finished
-        void* ctrl = nullptr;
-        if (failed(hipMalloc(&ctrl, sizeof(first)))) return false;
-        if (failed(hipMemcpy(ctrl, first, sizeof(first), hipMemcpyHostToDevice))) {
-            (void)hipFree(ctrl);
-            return false;
-        }
-        cs.ctrl = ctrl;
+    *out = &g_csync[dev];
+    return ELX_SUCCESS;
+}
+
+bool chain_area(ChainSync& cs, size_t bytes, hipStream_t s) {
+    if (cs.recorded && cs.bytes >= bytes) return true;
+    // another thread, or another stream of this one, may be capturing: allocations end a capture
+    // unless this thread's calls are exempt from it
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
     }
-    if (cs.bytes < bytes) {
+    auto ok = [](hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
+    };
+    auto get = [&]() {
+        if (!cs.last && !ok(hipEventCreateWithFlags(&cs.last, hipEventDisableTiming))) return false;
+        if (!cs.ctrl && !ok(hipMalloc(&cs.ctrl, kChainCtrl))) return false;
+        if (!cs.recorded) {
+            if (!ok(hipMemsetAsync(cs.ctrl, 0, kChainCtrl, s)) || !ok(hipEventRecord(cs.last, s))) return false;
+            cs.recorded = true;
+        }
+        if (cs.bytes >= bytes) return true;
         // the smaller area stays: queued launches may still use it, and uncached memory that a
         // kernel has read is not freed
         const size_t want = std::max<size_t>(std::max<size_t>(bytes, 2 * cs.bytes), (size_t)4 << 20);
         void* area = nullptr;
-        if (failed(hipExtMallocWithFlags(&area, want, hipDeviceMallocUncached))) return false;
+        if (!ok(hipExtMallocWithFlags(&area, want, hipDeviceMallocUncached))) return false;
         cs.area = area;
         cs.bytes = want;
-    }
-    return true;
+        return true;
+    };
+    const bool have = get();
+    (void)ok(hipThreadExchangeStreamCaptureMode(&mode));
+    return have;
 }
 
 // ---------------------------------------------------------------- kernel-class timing

@@ -91,19 +91,22 @@ struct RPanelSync {
 elx_status_t rpanel_sync_get(size_t bytes, RPanelSync** out);
 
 // The hand-off area of the chained triangular solves (solve_chain.hip): uncached memory, grown by
-// doubling and kept until the process ends, and the launch epoch in device memory. One launch at
-// a time uses it: a launch on another stream than the last one's first waits for `last`.
+// doubling and kept until the process ends, and the launch's control words in device memory. One
+// launch at a time uses it: every launch first waits for `last`, the event behind the one before
+// it, whatever their streams (an event knows its own stream: on the same one the wait costs
+// nothing). Captured launches never use it, a replay could not be ordered against the others.
+constexpr size_t kChainCtrl = 64;  // bytes of its control words
 struct ChainSync {
     void* area = nullptr;
     size_t bytes = 0;
     void* ctrl = nullptr;
-    hipEvent_t last = nullptr;  // recorded behind the last launch outside a capture
-    hipStream_t stream = nullptr;
+    hipEvent_t last = nullptr;
     bool recorded = false;
-    std::mutex mu;  // held from chain_sync_get's use to the launch
+    std::mutex mu;  // held from chain_area to the recording of `last`
 };
-// False where the area would have to be created or grown and cannot be (a capture, no memory).
-bool chain_sync_get(size_t bytes, bool capturing, ChainSync** out);
+elx_status_t chain_sync_get(ChainSync** out);
+// With cs.mu held: an area of at least `bytes` for a launch on s; false where it cannot be had.
+bool chain_area(ChainSync& cs, size_t bytes, hipStream_t s);
 
 inline unsigned cdiv(i64 a, i64 b) { return (unsigned)((a + b - 1) / b); }
 
@@ -194,7 +197,7 @@ elx_status_t launch_trsm_small_f32(hipStream_t s, int side, int uplo, int orient
 
 // Left triangular solve of any order with few right-hand sides, one persistent launch per 16 of
 // them (solve_chain.hip).
-// *taken = false, and nothing launched, where the hand-off area cannot be had.
+// *taken = false, and nothing launched, inside a capture and where the hand-off area cannot be had.
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
                                 const double* A, i64 lda, double* B, i64 ldb, const int32_t* stop, bool* taken);
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,

@@ -20,12 +20,11 @@
 // result is that of trsm_block_kernel and the GEMM kernels bit for bit.
 // The hand-off is through uncached memory in tagged 16-byte units (exchange.hpp): a unit holds
 // eight bytes of the solution, the launch's epoch and a hash, so a reader needs no flag or store
-// completion. The epoch lives in device memory and the last workgroup advances it, so replays of
-// a captured launch never take an earlier replay's units for their own. The area is one per
-// device, so launches from several streams wait for each other; where it cannot be had (a capture
-// that would have to allocate it, no memory left) the caller's blocked sequence runs instead. Each block waits only on
-// earlier blocks, which resident workgroups own; every wait is bounded, and a wait that runs out
-// turns the solution into NaN instead of hanging.
+// completion. The epoch lives in device memory and the last workgroup advances it. The area is one
+// per device and each launch waits for the one before it; inside a capture, and where the area
+// cannot be had, the caller's blocked sequence runs instead. Each block waits only on earlier
+// blocks, which resident workgroups own; every wait is bounded, and a wait that runs out turns the
+// solution into NaN instead of hanging.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -113,7 +112,7 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l16 = lane & 15, kq = lane >> 4;
     const int nblk = (int)((p.n + BS - 1) / BS);
-    const uint32_t epoch = p.ctrl[0];
+    const uint32_t epoch = p.ctrl[0] + 1u;  // never the tag of memory that is zero
     const i64 v0 = (i64)blockIdx.y * NV;
     const int nv = (int)((p.nrhs - v0) < NV ? (p.nrhs - v0) : NV);
     const uint32_t count = (uint32_t)nblk * UNITS;
@@ -327,7 +326,7 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
         const uint32_t total = gridDim.x * gridDim.y;
         if (atomicAdd(&p.ctrl[1], 1u) == total - 1) {
             p.ctrl[1] = 0u;
-            p.ctrl[0] = epoch + 1u;
+            p.ctrl[0] = epoch;
         }
     }
 }
@@ -341,16 +340,18 @@ elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i6
     const i64 most = std::min<i64>(MAX_GROUPS, (nrhs + NV - 1) / NV);
     ELX_ARG(units < ((size_t)1 << 27));
     *taken = false;
-    // a capture can neither allocate nor wait for an event from outside it; a status that cannot
-    // be had (another stream's capture forbids the call) counts as one
+    // Inside a capture the caller's blocked sequence runs: a replay on one stream could meet a solve
+    // on another, or a forked branch of its own graph, in the one hand-off area. A status that
+    // cannot be had (another stream's capture forbids the call) counts as a capture.
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     const hipError_t se = hipStreamIsCapturing(s, &st);
     if (se != hipSuccess) (void)hipGetLastError();
-    const bool capturing = se != hipSuccess || st != hipStreamCaptureStatusNone;
+    if (se != hipSuccess || st != hipStreamCaptureStatusNone) return ELX_SUCCESS;
     elx::ChainSync* sync = nullptr;
-    if (!elx::chain_sync_get(units * sizeof(u4) * (size_t)most, capturing, &sync)) return ELX_SUCCESS;
+    ELX_CHECK(elx::chain_sync_get(&sync));
     std::lock_guard<std::mutex> lk(sync->mu);
-    if (!capturing && sync->recorded && sync->stream != s) ELX_HIP(hipStreamWaitEvent(s, sync->last, 0));
+    if (!elx::chain_area(*sync, units * sizeof(u4) * (size_t)most, s)) return ELX_SUCCESS;
+    ELX_HIP(hipStreamWaitEvent(s, sync->last, 0));
     elx::ProfScope prof_(s, elx::kKTrsm, (double)n * (double)n * (double)nrhs);
     ChainArgs<T> a;
     a.n = n;
@@ -384,11 +385,7 @@ elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i6
         else ELX_CHECK(diag == elx::kUnit ? go(yes, four) : go(no, four));
         ELX_HIP(hipGetLastError());
     }
-    if (!capturing) {
-        ELX_HIP(hipEventRecord(sync->last, s));
-        sync->stream = s;
-        sync->recorded = true;
-    }
+    ELX_HIP(hipEventRecord(sync->last, s));
     *taken = true;
     return ELX_SUCCESS;
 }

@@ -113,3 +113,69 @@ def test_two_streams(dev):
     torch.cuda.synchronize()
     for dB in got:
         assert torch.equal(dB, want)
+
+
+def test_captured_branches_and_eager_solves_overlap(dev):
+    """Two forked branches of one capture, replayed while eager solves run on another stream."""
+    n = 1500
+    rng = np.random.default_rng(5)
+    dT = dev.to_device(np.tril(rng.standard_normal((n, n)) / n) + np.eye(n))
+    B = torch.from_numpy(rng.standard_normal((n, 2))).cuda()
+    want = dev.to_device(B.cpu().numpy())
+    dev.trsm(0, 0, 0, 0, 1.0, dT, want)
+    a, b = dev.colmajor_empty(n, 2), dev.colmajor_empty(n, 2)
+    eager = [dev.colmajor_empty(n, 2) for _ in range(6)]
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        cur = torch.cuda.current_stream()
+        side.wait_stream(cur)
+        dev.trsm(0, 0, 0, 0, 1.0, dT, a)
+        with torch.cuda.stream(side):
+            dev.trsm(0, 0, 0, 0, 1.0, dT, b)
+        cur.wait_stream(side)
+    for _ in range(4):
+        for t in [a, b] + eager:
+            t.copy_(B)
+        torch.cuda.synchronize()
+        g.replay()
+        with torch.cuda.stream(other):
+            for t in eager:
+                dev.trsm(0, 0, 0, 0, 1.0, dT, t)
+        torch.cuda.synchronize()
+        for t in [a, b] + eager:
+            assert torch.equal(t, want)
+
+
+def test_eager_solve_beside_a_capture(dev):
+    """An eager solve, the first of its size, on another stream while a capture is under way: the
+    capture stays valid and both solve."""
+    n, r = 12000, 128
+    dT = dev.colmajor_empty(n, n)
+    dT.copy_(torch.tril(torch.randn(n, n, dtype=torch.float64, device="cuda")) / n)
+    dT.diagonal().fill_(1.0)
+    small = dT[:700, :700]
+    B = torch.randn(n, r, dtype=torch.float64, device="cuda")
+    got, want, cap = dev.colmajor_empty(n, r), dev.colmajor_empty(n, r), dev.colmajor_empty(700, 2)
+    got.copy_(B)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        dev.trsm(0, 0, 0, 0, 1.0, small, cap)
+        with torch.cuda.stream(other):
+            dev.trsm(0, 0, 0, 0, 1.0, dT, got)
+        dev.trsm(0, 0, 1, 0, 1.0, small, cap)
+    torch.cuda.synchronize()
+    want.copy_(B)
+    dev.trsm(0, 0, 0, 0, 1.0, dT, want)
+    assert torch.equal(got, want)
+    ref = dev.to_device(B[:700, :2].cpu().numpy())
+    dev.trsm(0, 0, 0, 0, 1.0, small, ref)
+    dev.trsm(0, 0, 1, 0, 1.0, small, ref)
+    for _ in range(3):
+        cap.copy_(B[:700, :2])
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(cap, ref)
