@@ -348,7 +348,7 @@ constexpr i64 kChainRhs = 128;
 template <typename T>
 elx_status_t trsm_blocked(hipStream_t s, int side, int uplo, int orient, int diag, i64 m, i64 n,
                           T alpha, const T* A, i64 lda, T* B, i64 ldb,
-                          const int32_t* stop = nullptr, bool allow_library = true,
+                          int32_t* stop = nullptr, bool allow_library = true,
                           bool dot_order = false) {
     if (m <= 0 || n <= 0) return ELX_SUCCESS;
     if (alpha != T(1))

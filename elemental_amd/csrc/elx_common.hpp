@@ -197,11 +197,12 @@ elx_status_t launch_trsm_small_f32(hipStream_t s, int side, int uplo, int orient
 
 // Left triangular solve of any order with few right-hand sides, one persistent launch per 16 of
 // them (solve_chain.hip).
-// *taken = false, and nothing launched, inside a capture and where the hand-off area cannot be had.
+// info (may be null): non-zero stops the solve, and a wait between workgroups that runs out sets it
+// to -1. *taken = false, and nothing launched, inside a capture and where the hand-off area cannot be had.
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
-                                const double* A, i64 lda, double* B, i64 ldb, const int32_t* stop, bool* taken);
+                                const double* A, i64 lda, double* B, i64 ldb, int32_t* info, bool* taken);
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
-                                const float* A, i64 lda, float* B, i64 ldb, const int32_t* stop, bool* taken);
+                                const float* A, i64 lda, float* B, i64 ldb, int32_t* info, bool* taken);
 
 // General triangular solve (blocked by 128 with GEMM updates for larger triangles).
 elx_status_t dtrsm(hipStream_t s, int side, int uplo, int orient, int diag, i64 m, i64 n,

@@ -6,7 +6,7 @@
 // a diagonal solve and a GEMM per 128 rows: at 1 to 16 columns each of those kernels was one
 // dependent chain on a mostly idle chip (20-38 us for the diagonal block, 29 us for an update
 // whose 128 x 128 tiles held 1 to 16 used columns), 256 pairs of them in an n = 16384 solve.
-// Here workgroup g owns the 128-row blocks g, g + G, ...; a block's rows take the products with
+// Here a workgroup takes one 128-row block after another; a block's rows take the products with
 // the earlier blocks' solutions as those are published, then the block's triangle is solved 16
 // rows at a time: wave w holds rows 16 w .. 16 w + 15 of all 16 vectors in one MFMA accumulator,
 // wave s solves its 16 x 16 triangle, and the waves below it update on the matrix cores. What
@@ -22,10 +22,14 @@
 // eight bytes of the solution, the launch's epoch and a hash, so a reader needs no flag or store
 // completion. The epoch lives in device memory and the last workgroup advances it. The area is one
 // per device and each launch waits for the one before it; inside a capture, and where the area
-// cannot be had, the caller's blocked sequence runs instead. Each block waits only on earlier
-// blocks, which resident workgroups own; every wait is bounded, and a wait that runs out turns the
-// solution into NaN instead of hanging.
+// cannot be had, the caller's blocked sequence runs instead.
+// The blocks are dealt out in order by a counter, so a block waits only on blocks that running
+// workgroups hold, never on one that has yet to get its place on the chip, whatever else runs
+// there. Every wait is bounded all the same (ELX_SOLVE_SPIN_LIMIT polls, 2^20 unless set, some
+// seconds): one that runs out turns the solution into NaN and, where the caller has an info word,
+// that into -1.
 #include <algorithm>
+#include <cstdlib>
 #include <mutex>
 #include <type_traits>
 
@@ -44,7 +48,7 @@ namespace {
 constexpr int BS = 128, SB = 16, NW = BS / SB, CNT = 64 * NW;  // block, sub-block, waves, threads
 constexpr int NV = 16;                                         // right-hand sides per group
 constexpr int MAX_GROUPS = 8;
-constexpr int SPIN_LIMIT = 1 << 20;
+constexpr int SPIN_LIMIT = 1 << 20;  // polls of a wait
 
 // Eight bytes of a row of the solution: entries PER*q .. of its 16 vectors.
 template <typename T>
@@ -82,9 +86,11 @@ struct ChainArgs {
     T* B;
     i64 ldb;
     int mtrans, back;
-    const int32_t* stop;
+    int32_t* info;   // may be null: non-zero stops the solve, a wait that runs out sets -1
     u4* area;        // [groups][nblk][BS * NV / PER] units
-    uint32_t* ctrl;  // epoch, workgroups finished
+    uint32_t* ctrl;  // epoch, workgroups finished, blocks dealt out, waits lost
+    int groups;      // of 16 right-hand sides
+    int spin_limit;
 };
 
 // The exchange loads are plain intrinsics to the compiler: without this a poll loop's load could
@@ -108,15 +114,13 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
     __shared__ T xs[2][BS * NV];           // an earlier block's solution, [k][v]
     __shared__ T xd[BS][NV + 1];           // this block's
     __shared__ T tiles[NW][SB][SB + 1];
-    if (p.stop && *p.stop != 0) return;
+    __shared__ uint32_t s_item;
+    if (p.info && *p.info != 0) return;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l16 = lane & 15, kq = lane >> 4;
     const int nblk = (int)((p.n + BS - 1) / BS);
     const uint32_t epoch = p.ctrl[0] + 1u;  // never the tag of memory that is zero
-    const i64 v0 = (i64)blockIdx.y * NV;
-    const int nv = (int)((p.nrhs - v0) < NV ? (p.nrhs - v0) : NV);
     const uint32_t count = (uint32_t)nblk * UNITS;
-    const u4* area = p.area + (size_t)blockIdx.y * count;
     // Logical forward problem: the backward forms walk both matrices from their ends, over the
     // same 128-row blocks from the top (so the partial block comes first: rows before lo do not
     // exist and are those of the identity).
@@ -124,7 +128,6 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
     const i64 lo = p.back ? np - p.n : 0, hi = p.back ? np : p.n;
     const i64 si = sgn * (p.mtrans ? p.lda : 1), sj = sgn * (p.mtrans ? 1 : p.lda), ei = sgn;
     const T* __restrict__ M0 = p.back ? p.A - (np - 1) * (si + sj) : p.A;
-    T* X0 = (p.back ? p.B - (np - 1) * ei : p.B) + v0 * p.ldb;
     // within an earlier block the products go up the matrix's own columns either way
     const int kfirst = p.back ? BS - 1 - kq : kq;
     const i64 sk = p.back ? -sj : sj;
@@ -132,7 +135,17 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
     auto vcol = [&](int r) { return kq + 4 * r; };
     bool lost = false;
 
-    for (int b = blockIdx.x; b < nblk; b += gridDim.x) {
+    for (;;) {
+        // the next block, the groups of right-hand sides side by side
+        if (t == 0) s_item = atomicAdd(&p.ctrl[2], 1u);
+        __syncthreads();
+        const int item = __builtin_amdgcn_readfirstlane((int)s_item);
+        if (item >= nblk * p.groups) break;
+        const int b = item / p.groups, group = item - b * p.groups;
+        const i64 v0 = (i64)group * NV;
+        const int nv = (int)((p.nrhs - v0) < NV ? (p.nrhs - v0) : NV);
+        const u4* area = p.area + (size_t)group * count;
+        T* X0 = (p.back ? p.B - (np - 1) * ei : p.B) + v0 * p.ldb;
         const i64 i0 = (i64)b * BS, iw = i0 + SB * wave;  // the block's and this wave's first row
         const i64 il = iw + l16;
         const bool rin = il >= lo && il < hi;
@@ -183,7 +196,7 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
             int spins = 0;
             // one lane per wave watches the block's last unit, then every thread reads its own
             if (lane == 0 && !lost) {
-                while (ld16(area, count, at + UNITS - 1)[2] != epoch && spins < SPIN_LIMIT) {
+                while (ld16(area, count, at + UNITS - 1)[2] != epoch && spins < p.spin_limit) {
                     ++spins;
                     reread();
                 }
@@ -208,7 +221,7 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
                     all = all && got[u];
                 }
                 if (__all(all ? 1 : 0)) break;
-                if (lost || ++spins > SPIN_LIMIT) {
+                if (lost || ++spins > p.spin_limit) {
                     lost = true;
 #pragma unroll
                     for (int u = 0; u < UPT; ++u)
@@ -320,20 +333,24 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
         }
         __syncthreads();
     }
-    // the last workgroup to finish opens the next launch's epoch
+    // the last workgroup to finish opens the next launch's epoch and its count of blocks, and reports a
+    // lost wait (not before: a workgroup that starts late still has to find the info word as it was)
+    if (lost && lane == 0) {
+        atomicOr(&p.ctrl[3], 1u);
+        __threadfence();
+    }
     __syncthreads();
-    if (t == 0) {
-        const uint32_t total = gridDim.x * gridDim.y;
-        if (atomicAdd(&p.ctrl[1], 1u) == total - 1) {
-            p.ctrl[1] = 0u;
-            p.ctrl[0] = epoch;
-        }
+    if (t == 0 && atomicAdd(&p.ctrl[1], 1u) == gridDim.x - 1) {
+        if (atomicExch(&p.ctrl[3], 0u) != 0u && p.info) *p.info = -1;
+        p.ctrl[1] = 0u;
+        p.ctrl[2] = 0u;
+        p.ctrl[0] = epoch;
     }
 }
 
 template <typename T>
 elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs, const T* A, i64 lda,
-                        T* B, i64 ldb, const int32_t* stop, bool* taken) {
+                        T* B, i64 ldb, int32_t* info, bool* taken) {
     const elx::DeviceInfo& di = elx::device_info();
     const i64 nblk = (n + BS - 1) / BS;
     const size_t units = (size_t)nblk * (BS * NV / Unit<T>::PER);
@@ -360,29 +377,28 @@ elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i6
     a.ldb = ldb;
     a.mtrans = orient != elx::kNormal ? 1 : 0;
     a.back = ((uplo == elx::kLower) != (a.mtrans != 0)) ? 0 : 1;
-    a.stop = stop;
+    a.info = info;
+    const char* limit = std::getenv("ELX_SOLVE_SPIN_LIMIT");
+    a.spin_limit = limit ? std::min(std::max(std::atoi(limit), 0), 1 << 30) : SPIN_LIMIT;
     a.area = static_cast<u4*>(sync->area);
     a.ctrl = static_cast<uint32_t*>(sync->ctrl);
     for (i64 v = 0; v < nrhs; v += NV * MAX_GROUPS) {
         a.nrhs = std::min<i64>(nrhs - v, NV * MAX_GROUPS);
         a.B = B + v * ldb;
         const i64 groups = (a.nrhs + NV - 1) / NV;
-        const i64 G = std::max<i64>(1, std::min<i64>(nblk, di.num_cus / groups));
-        const dim3 grid((unsigned)G, (unsigned)groups);
-        auto go = [&](auto ut, auto rt) -> elx_status_t {
+        const dim3 grid((unsigned)std::min<i64>(nblk * groups, di.num_cus));
+        a.groups = (int)groups;
+        auto go = [&](auto ut, auto rt) {
             constexpr bool U = decltype(ut)::value;
             constexpr int R = decltype(rt)::value;
-            ELX_CHECK(elx::coop_fits(reinterpret_cast<const void*>(&solve_chain_kernel<T, U, R>), CNT, 0,
-                                     G * groups));
             hipLaunchKernelGGL((solve_chain_kernel<T, U, R>), grid, dim3(CNT), 0, s, a);
-            return ELX_SUCCESS;
         };
         const std::integral_constant<int, 1> one;
         const std::integral_constant<int, 4> four;
         const std::true_type yes;
         const std::false_type no;
-        if (a.nrhs <= 4) ELX_CHECK(diag == elx::kUnit ? go(yes, one) : go(no, one));
-        else ELX_CHECK(diag == elx::kUnit ? go(yes, four) : go(no, four));
+        if (a.nrhs <= 4) diag == elx::kUnit ? go(yes, one) : go(no, one);
+        else diag == elx::kUnit ? go(yes, four) : go(no, four);
         ELX_HIP(hipGetLastError());
     }
     ELX_HIP(hipEventRecord(sync->last, s));
@@ -395,14 +411,14 @@ elx_status_t chain_impl(hipStream_t s, int uplo, int orient, int diag, i64 n, i6
 namespace elx {
 
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
-                                const double* A, i64 lda, double* B, i64 ldb, const int32_t* stop,
+                                const double* A, i64 lda, double* B, i64 ldb, int32_t* info,
                                 bool* taken) {
-    return chain_impl<double>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, stop, taken);
+    return chain_impl<double>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, info, taken);
 }
 elx_status_t launch_solve_chain(hipStream_t s, int uplo, int orient, int diag, i64 n, i64 nrhs,
-                                const float* A, i64 lda, float* B, i64 ldb, const int32_t* stop,
+                                const float* A, i64 lda, float* B, i64 ldb, int32_t* info,
                                 bool* taken) {
-    return chain_impl<float>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, stop, taken);
+    return chain_impl<float>(s, uplo, orient, diag, n, nrhs, A, lda, B, ldb, info, taken);
 }
 
 }  // namespace elx

@@ -17,8 +17,11 @@
  *                    reference leaves them when it throws.
  *   *dInfo == -1     the LU panel gave up waiting for a peer workgroup (a GPU shared with
  *                    other work can delay one); A is unchanged from the start of that panel
- *                    (its current 32-column block) on. A runtime error, not a numerical
- *                    result.
+ *                    (its current 32-column block) on. Or (gesv, posv) the solve
+ *                    that follows the factorization did; then B holds NaN. A runtime error,
+ *                    not a numerical result. A lost wait of getrs, potrs and trsm, which have
+ *                    no info word, leaves NaN in B; it takes a running workgroup that stands
+ *                    still for seconds.
  * Block sizes nb > 128 run as 128-column panels (the same pivots in exact arithmetic).
  *
  * Every routine of the plain path exists for FP64 (elx_d*) and FP32 (elx_s*), as the

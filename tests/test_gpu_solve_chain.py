@@ -179,3 +179,48 @@ def test_eager_solve_beside_a_capture(dev):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(cap, ref)
+
+
+def test_a_wait_that_runs_out_is_reported(dev, monkeypatch):
+    """With no poll allowed the blocks give up on each other: gesv and posv say so in their info word,
+    and the next solves are whole again."""
+    n = 2000
+    rng = np.random.default_rng(6)
+    A = rng.standard_normal((n, n))
+    H = A @ A.T / n + np.eye(n)
+    B = rng.standard_normal((n, 3))
+
+    def solve():
+        x, y = dev.to_device(B), dev.to_device(B)
+        infos = [dev.gesv(dev.to_device(A), x), dev.posv(dev.to_device(H), y)]
+        return [int(i.item()) for i in infos], x, y
+
+    first, x0, y0 = solve()
+    assert first == [0, 0]
+    monkeypatch.setenv("ELX_SOLVE_SPIN_LIMIT", "0")
+    lost, x, y = solve()
+    assert lost == [-1, -1]
+    assert bool(torch.isnan(x).any()) and bool(torch.isnan(y).any())
+    monkeypatch.delenv("ELX_SOLVE_SPIN_LIMIT")
+    again, x, y = solve()
+    assert again == [0, 0] and torch.equal(x, x0) and torch.equal(y, y0)
+
+
+@pytest.mark.parametrize("n,nrhs", [(128 * 256 + 1, 1), (128 * 40, 128)])
+def test_more_blocks_than_workgroups(dev, n, nrhs):
+    """Workgroups that take several blocks each, against a solve of the same system block by block
+    (more than 128 columns): bit for bit."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    dT = dev.colmajor_empty(n, n, torch.float32)
+    dT.copy_(torch.randn(n, n, dtype=torch.float32, device="cuda", generator=g) / n)
+    dT.diagonal().add_(1.0)
+    B = torch.randn(n, nrhs, dtype=torch.float32, device="cuda", generator=g)
+    for uplo in (0, 1):
+        wide, got = dev.colmajor_empty(n, 130, torch.float32), dev.colmajor_empty(n, nrhs, torch.float32)
+        wide.zero_()
+        wide[:, :nrhs] = B
+        got.copy_(B)
+        dev.trsm(0, uplo, 0, 0, 1.0, dT, wide)
+        dev.trsm(0, uplo, 0, 0, 1.0, dT, got)
+        assert torch.equal(got, wide[:, :nrhs])
