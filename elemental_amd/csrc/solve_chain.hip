@@ -97,15 +97,6 @@ struct ChainArgs {
 // be taken out of the loop.
 __device__ __forceinline__ void reread() { asm volatile("" ::: "memory"); }
 
-// x / d for |d| well inside the exponent range, r = 1 / d correctly rounded: one correction step
-// of x r. An infinite or NaN correction (x or r not finite) leaves x r.
-template <typename T>
-__device__ __forceinline__ T quot(T x, T d, T r) {
-    const T q = x * r;
-    const T c = __builtin_fma(__builtin_fma(-q, d, x), r, q);
-    return finite(c) ? c : q;
-}
-
 // NR: vectors per lane in a triangle solve: 4, or 1 where the group has at most 4 vectors.
 template <typename T, bool UNIT, int NR>
 __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
@@ -253,11 +244,6 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
         // they are solved (one barrier each), solves its own and publishes it while the waves
         // below go on
         const T dr = UNIT ? T(1) : T(1) / dg;
-        bool plain = false;  // a diagonal entry outside the range of quot()
-        if (!UNIT) {
-            const double m = fabs((double)dg), lim = sizeof(T) == 8 ? 1e290 : 1e30;
-            plain = !__all((m < lim && m > 1.0 / lim) ? 1 : 0);
-        }
         const int nsub = (int)((hi - i0 < BS ? hi - i0 : BS) + SB - 1) / SB;
         static_for<0, NW - 1>([&](auto sc) {
             constexpr int s = decltype(sc)::value;
@@ -274,35 +260,38 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) tile[MF::row(kq, r)][l16] = acc[r];
             wave_lds_sync();
+            // every lane divides its entry at each step; the step's own is lane k's, whose entry is
+            // final but for that division
+            auto solve = [&](auto divide) {
 #pragma unroll
-            for (int r = 0; r < NR; ++r) x[r] = tile[l16][vcol(r)];
-            static_for<0, SB>([&](auto kc) {
-                constexpr int k = decltype(kc)::value;
-                T xk[NR];
-                if constexpr (UNIT) {
+                for (int r = 0; r < NR; ++r) x[r] = tile[l16][vcol(r)];
+                static_for<0, SB>([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    T xk[NR];
 #pragma unroll
-                    for (int r = 0; r < NR; ++r) xk[r] = row_bcast<k>(x[r]);
+                    for (int r = 0; r < NR; ++r) xk[r] = row_bcast<k>(divide(x[r]));
+                    if (l16 > k) {
+#pragma unroll
+                        for (int r = 0; r < NR; ++r) x[r] = __builtin_fma(-mrow[k], xk[r], x[r]);
+                    }
+                });
+            };
+            if constexpr (UNIT) {
+                solve([](T v) { return v; });
+            } else {
+                solve([&](T v) { return quot(v, dg, dr); });
+                bool ok = divisor_ok(dg);
+#pragma unroll
+                for (int r = 0; r < NR; ++r) ok = ok && dividend_ok(x[r]);
+                if (__all(ok ? 1 : 0)) {
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) x[r] = quot(x[r], dg, dr);
                 } else {
-                    // every lane divides its entry; the final one is lane k's
-                    T y[NR];
-                    if (!plain) {
+                    solve([&](T v) { return v / dg; });
 #pragma unroll
-                        for (int r = 0; r < NR; ++r) y[r] = quot(x[r], dg, dr);
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < NR; ++r) y[r] = x[r] / dg;
-                    }
-#pragma unroll
-                    for (int r = 0; r < NR; ++r) {
-                        xk[r] = row_bcast<k>(y[r]);
-                        if (l16 == k) x[r] = y[r];
-                    }
+                    for (int r = 0; r < NR; ++r) x[r] = x[r] / dg;
                 }
-                if (l16 > k) {
-#pragma unroll
-                    for (int r = 0; r < NR; ++r) x[r] = __builtin_fma(-mrow[k], xk[r], x[r]);
-                }
-            });
+            }
 #pragma unroll
             for (int r = 0; r < NR; ++r) xd[SB * wave + l16][vcol(r)] = x[r];
             if (NR < 4) {

@@ -42,6 +42,28 @@ __device__ __forceinline__ void static_for(F&& f) {
         static_for<I + 1, N>(f);
     }
 }
+
+// x / d by the reciprocal r = 1 / d: x r and one correction with the exact remainder, then rounded
+// as the division rounds it (compared with it on the quotients that lie closest to a rounding
+// boundary, for every FP32 divisor). That holds where nothing leaves the exponent range on the way:
+// divisor_ok(d) and dividend_ok(x). A zero x keeps the quotient's sign.
+__device__ __forceinline__ double quot(double x, double d, double r) {
+    const double q = x * r;
+    return __builtin_copysign(__builtin_fma(__builtin_fma(-q, d, x), r, q), q);
+}
+__device__ __forceinline__ float quot(float x, float d, float r) {
+    const float q = x * r;
+    return __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-q, d, x), r, q), q);
+}
+__device__ __forceinline__ bool divisor_ok(double d) { return fabs(d) <= 0x1p400 && fabs(d) >= 0x1p-400; }
+__device__ __forceinline__ bool divisor_ok(float d) { return fabsf(d) <= 0x1p60f && fabsf(d) >= 0x1p-60f; }
+__device__ __forceinline__ bool dividend_ok(double x) {
+    return x == 0.0 || (fabs(x) <= 0x1p600 && fabs(x) >= 0x1p-600);
+}
+__device__ __forceinline__ bool dividend_ok(float x) {
+    return x == 0.0f || (fabsf(x) <= 0x1p64f && fabsf(x) >= 0x1p-64f);
+}
+
 __device__ __forceinline__ bool finite(double v) { return fabs(v) <= 1.7976931348623157e308; }
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.4028234663852886e38f; }
 

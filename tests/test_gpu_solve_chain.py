@@ -224,3 +224,36 @@ def test_more_blocks_than_workgroups(dev, n, nrhs):
         dev.trsm(0, uplo, 0, 0, 1.0, dT, wide)
         dev.trsm(0, uplo, 0, 0, 1.0, dT, got)
         assert torch.equal(got, wide[:, :nrhs])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_divisions_at_the_ends_of_the_range(dev, dtype):
+    """Right-hand sides near underflow and overflow, signed zeros and infinities, and divisors far from 1:
+    the chained solve divides as the block by block one (more than 128 columns) does, bit for bit."""
+    n = 300
+    rng = np.random.default_rng(7)
+    tiny, top = (-1060, 1020) if dtype == np.float64 else (-140, 125)
+    exps = [tiny, tiny + 15, tiny + 30, tiny // 2, 0, top // 2, top - 20, top]
+    B = np.stack([np.ldexp(rng.standard_normal(n), e) for e in exps] +
+                 [np.zeros(n), -np.zeros(n), np.ldexp(rng.standard_normal(n), rng.integers(tiny, top, n))],
+                 axis=1).astype(dtype)
+    B[:, 10][rng.integers(0, n, 20)] = -0.0
+    B = np.concatenate([B, B[:, 4:6]], axis=1)
+    B[200, 11] = np.inf
+    for spread in (0, 55, tiny // -2):
+        T = np.tril(rng.standard_normal((n, n)) / n)
+        T[np.arange(n), np.arange(n)] = np.ldexp(1.0 + rng.random(n), rng.integers(-spread, spread + 1, n))
+        T[np.arange(0, n, 3), np.arange(0, n, 3)] *= -1
+        dT = dev.to_device(T.astype(dtype))
+        wide = np.zeros((n, 130), dtype)
+        wide[:, :B.shape[1]] = B
+        for orient in (0, 1):
+            for cols in (3, B.shape[1]):
+                dB, dW = dev.to_device(np.ascontiguousarray(B[:, :cols])), dev.to_device(wide)
+                dev.trsm(0, 0, orient, 0, 1.0, dT, dB)
+                dev.trsm(0, 0, orient, 0, 1.0, dT, dW)
+                x, y = dev.to_host(dB), dev.to_host(dW)[:, :cols]
+                bits = np.int64 if dtype == np.float64 else np.int32
+                same = (x.view(bits) == y.view(bits)) | (np.isnan(x) & np.isnan(y))
+                print("[case]", dtype.__name__, spread, orient, cols, int((~same).sum()), flush=True)
+                assert same.all()
