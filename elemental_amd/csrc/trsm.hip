@@ -23,10 +23,12 @@ namespace {
 // broadcast), x goes through the wave's own LDS tile into operand layout, and the later blocks
 // are updated on the matrix cores, whose products are the same FMA chains in the same order,
 // so the results are the scalar code's bit for bit. No workgroup barrier; the triangle is read
-// straight from the caches in operand layout. What bounds it: per wave 8 dependent block solves
-// of 16 steps and 28 tile products, FP64 17-27 us (right side) and 11-24 us (left, unit
-// diagonal) from 64 to 16384 vectors, one wave per SIMD; with 16 lanes per vector, all 128 steps
-// dependent and 132 KB of LDS per 16 vectors, it took 52 us per 4096 vectors (240 us at 16256).
+// straight from the caches in operand layout. Divisions are quotients by the reciprocal where the
+// operands allow it (wave.hpp), else the block is solved again with plain ones. What bounds it: per
+// wave 8 dependent block solves of 16 steps and 28 tile products, FP64 17-27 us (right side), 11-24
+// us (left, unit diagonal) and, left and non-unit, 15 us for one vector (23 with plain divisions, 20
+// with 16 lanes per vector), one wave per SIMD; with 16 lanes per vector, all 128 steps dependent and
+// 132 KB of LDS per 16 vectors, it took 52 us per 4096 vectors (240 us at 16256).
 //
 // maxbits (may be null): the largest |entry| written is folded into *maxbits (the bits of a
 // non-negative float, atomic max), for the exponent of a low-precision product that follows.
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
         constexpr int b = decltype(bc)::value, p = b & 1;
         if (FULL || TBLK * b < m) {
             if constexpr (b + 1 < TNB) load(std::integral_constant<int, b + 1>{});
-            const T dg = (RIGHT && !UNIT) ? T(1) / dgv[p] : dgv[p];
+            const T dg = dgv[p], dr = UNIT ? T(1) : T(1) / dg;
             // S(v, i): lane l16 holds entry i, register r vector MF::row(kq, r)
             T x[4];
             if (RIGHT) {
@@ -106,24 +108,41 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
 #pragma unroll
                 for (int r = 0; r < 4; ++r) x[r] = acc[b][r];
             }
-            // a lane's entry is final (but for its own diagonal) once the earlier ones are applied
-            static_for<0, TBLK>([&](auto kc) {
-                constexpr int k = decltype(kc)::value;
-                const T dk = UNIT ? T(1) : row_bcast<k>(dg);
-                T xk[4];
+            // a lane's entry is final (but for its own diagonal) once the earlier ones are applied;
+            // every lane scales its entry at each step, and the step's own is lane k's
+            auto substitute = [&](auto scale) {
+                static_for<0, TBLK>([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    T xk[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    xk[r] = row_bcast<k>(x[r]);
-                    if (!UNIT) xk[r] = RIGHT ? xk[r] * dk : xk[r] / dk;
+                    for (int r = 0; r < 4; ++r) xk[r] = row_bcast<k>(scale(x[r]));
+                    if (l16 > k) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) x[r] = __builtin_fma(-mrow[p][k], xk[r], x[r]);
+                    }
+                });
+            };
+            if constexpr (UNIT) {
+                substitute([](T v) { return v; });
+            } else if constexpr (RIGHT) {
+                substitute([&](T v) { return v * dr; });
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[r] = x[r] * dr;
+            } else {
+                substitute([&](T v) { return quot(v, dg, dr); });
+                bool ok = divisor_ok(dg);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ok = ok && dividend_ok(x[r]);
+                if (__all(ok ? 1 : 0)) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[r] = quot(x[r], dg, dr);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[r] = acc[b][r];
+                    substitute([&](T v) { return v / dg; });
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[r] = x[r] / dg;
                 }
-                if (l16 > k) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = __builtin_fma(-mrow[p][k], xk[r], x[r]);
-                }
-            });
-            if (!UNIT) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) x[r] = RIGHT ? x[r] * dg : x[r] / dg;
             }
             if (maxbits) {
 #pragma unroll
@@ -163,36 +182,108 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
 }
 
 // The transposed backward forms as the reference BLAS computes them: each x_i a dot product in
-// ascending k from its nearest entry on, which is one dependent chain per vector. A thread per
-// vector, the vectors in LDS. Only a direct Trsm of order <= 128 asks for this order; the solves
-// of larger systems and of factored ones run their diagonal blocks through trsm_block_kernel.
-constexpr int DNT = 64;  // vectors per workgroup
+// ascending k from its nearest entry on, which is one dependent chain per vector, m (m - 1) / 2 FMAs
+// and m quotients. Four waves bring the triangle (packed by its rows) and the vectors to LDS, then
+// one wave solves, a vector per lane: 16 rows at a time, their solutions and those of the next 16
+// in registers, the operands read ahead of the chain. Columns past the order are zero and so are their
+// unknowns: such terms leave a sum as it is. Left, unit, 64 vectors: order 64 47 us (FP64) and 56
+// (FP32), order 128 124 and 156 us; with each row fetched through the scalar cache as its step began
+// 84, 88, 222 and 233, and with 16 lanes per vector 69, 120, 210 and 410.
+// Only a direct Trsm of order <= 128 asks for this order; the solves of larger systems and of
+// factored ones run their diagonal blocks through trsm_block_kernel.
+constexpr int DNT = 64, DB = 16;  // vectors per workgroup, rows per block
 template <typename T>
-__global__ __launch_bounds__(DNT) void trsm_dot_kernel(int m, i64 nvec, const T* __restrict__ A, i64 lda,
+__global__ __launch_bounds__(256) void trsm_dot_kernel(int m, i64 nvec, const T* __restrict__ A, i64 lda,
                                                        T* B, i64 ldb, int right, int unit,
                                                        const int32_t* __restrict__ stop) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* xs = reinterpret_cast<T*>(smem_raw);  // xs[i * DNT + v]
+    const int nb = (m + DB - 1) / DB, mp = nb * DB;
+    T* xs = reinterpret_cast<T*>(smem_raw);  // xs[i * DNT + v], mp rows
+    T* tri = xs + mp * DNT;                  // M(i, k) = A(k, i), k >= i, at row(i)[k]
+    auto row = [&](int i) { return tri + (i * mp - i * (i - 1) / 2 - i); };
+    T* inv = tri + mp * (mp + 1) / 2;        // 1 / M(i, i)
     if (stop && *stop != 0) return;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const i64 v0 = (i64)blockIdx.x * DNT;
     const int nv = (int)((nvec - v0) < DNT ? (nvec - v0) : DNT);
+#pragma unroll 4
+    for (int i = wave; i < m; i += 4)
+        for (int k = i + lane; k < mp; k += 64) row(i)[k] = k < m ? A[k + i * lda] : T(0);
+    if (!unit && t < m) inv[t] = T(1) / A[t + t * lda];
     // a vector per lane (right) or down the columns (left): coalesced either way
-    for (int idx = t; idx < m * DNT; idx += DNT) {
-        const int i = right ? idx / DNT : idx % m, v = right ? idx % DNT : idx / m;
-        xs[i * DNT + v] = v < nv ? (right ? B[v0 + v + (i64)i * ldb] : B[i + (v0 + v) * ldb]) : T(0);
+#pragma unroll 4
+    for (int idx = t; idx < mp * DNT; idx += 256) {
+        const int i = right ? idx / DNT : idx % mp, v = right ? idx % DNT : idx / mp;
+        xs[i * DNT + v] = (v < nv && i < m) ? (right ? B[v0 + v + (i64)i * ldb] : B[i + (v0 + v) * ldb]) : T(0);
     }
     __syncthreads();
-    for (int i = m - 1; i >= 0; --i) {
-        const T* row = A + i * lda;  // M(i, k) = A(k, i)
-        T temp = xs[i * DNT + t];
-#pragma unroll 8
-        for (int k = i + 1; k < m; ++k) temp = __builtin_fma(-row[k], xs[k * DNT + t], temp);
-        if (!unit) temp = right ? temp * (T(1) / row[i]) : temp / row[i];
-        xs[i * DNT + t] = temp;
+    if (wave == 0) {
+        T xi[DB], xn[DB];               // this block's solutions and the next one's
+        T ri[DB], rn[DB], bi, dr;       // a row's entries beside them, its right-hand side and inverse diagonal
+        T xb[2][DB], rb[2][DB];         // blocks further on
+        auto row_ahead = [&](int i, bool more) __attribute__((always_inline)) {
+            const T* r = row(i);
+            const int k0 = i / DB * DB;
+            bi = xs[i * DNT + t];
+            if (!unit) dr = inv[i];
+#pragma unroll
+            for (int u = 0; u < DB; ++u) ri[u] = r[k0 + u];  // those left of the diagonal are not used
+            if (more) {
+#pragma unroll
+                for (int u = 0; u < DB; ++u) rn[u] = r[k0 + DB + u];
+            }
+        };
+        row_ahead(m - 1, false);
+        for (int ib = nb - 1; ib >= 0; --ib) {
+            const bool more = ib + 1 < nb;
+            static_for<0, DB>([&](auto rc) __attribute__((always_inline)) {
+                constexpr int r = DB - 1 - decltype(rc)::value;
+                const int i = ib * DB + r;
+                if (i >= m) {
+                    xi[r] = T(0);
+                    return;
+                }
+                const T* rp = row(i);
+                auto fetch = [&](int kb, T(&x)[DB], T(&w)[DB]) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int u = 0; u < DB; ++u) {
+                        x[u] = xs[(kb * DB + u) * DNT + t];
+                        w[u] = rp[kb * DB + u];
+                    }
+                };
+                T acc = bi;
+                const T d = ri[r], di = dr;
+                if (ib + 2 < nb) fetch(ib + 2, xb[0], rb[0]);
+#pragma unroll
+                for (int u = r + 1; u < DB; ++u) acc = __builtin_fma(-ri[u], xi[u], acc);
+                if (more) {
+#pragma unroll
+                    for (int u = 0; u < DB; ++u) acc = __builtin_fma(-rn[u], xn[u], acc);
+                }
+                if (i > 0) row_ahead(i - 1, r > 0 ? more : true);
+                for (int kb = ib + 2; kb < nb; kb += 2) {
+                    if (kb + 1 < nb) fetch(kb + 1, xb[1], rb[1]);
+#pragma unroll
+                    for (int u = 0; u < DB; ++u) acc = __builtin_fma(-rb[0][u], xb[0][u], acc);
+                    if (kb + 1 >= nb) break;
+                    if (kb + 2 < nb) fetch(kb + 2, xb[0], rb[0]);
+#pragma unroll
+                    for (int u = 0; u < DB; ++u) acc = __builtin_fma(-rb[1][u], xb[1][u], acc);
+                }
+                if (!unit) {
+                    if (right) acc = acc * di;
+                    else if (__all(divisor_ok(d) && dividend_ok(acc) ? 1 : 0)) acc = quot(acc, d, di);
+                    else acc = acc / d;
+                }
+                xi[r] = acc;
+                xs[i * DNT + t] = acc;
+            });
+#pragma unroll
+            for (int u = 0; u < DB; ++u) xn[u] = xi[u];
+        }
     }
     __syncthreads();
-    for (int idx = t; idx < m * DNT; idx += DNT) {
+    for (int idx = t; idx < m * DNT; idx += 256) {
         const int i = right ? idx / DNT : idx % m, v = right ? idx % DNT : idx / m;
         if (v < nv) {
             if (right) B[v0 + v + (i64)i * ldb] = xs[i * DNT + v];
@@ -223,8 +314,17 @@ static elx_status_t trsm_small_impl(hipStream_t s, int side, int uplo, int orien
     const int unit = diag == kUnit ? 1 : 0, mt = mtrans ? 1 : 0;
     ProfScope prof_(s, kKTrsm, (double)order * (double)order * (double)nvec);
     if (!lower_eff && mtrans && dot_order) {
-        hipLaunchKernelGGL(trsm_dot_kernel<T>, dim3(cdiv(nvec, DNT)), dim3(DNT),
-                           sizeof(T) * (size_t)order * DNT, s, (int)order, nvec, A, lda, B, ldb, right ? 1 : 0, unit, stop);
+        auto bytes = [](size_t m) {
+            m = (m + DB - 1) / DB * DB;
+            return sizeof(T) * (m * DNT + m * (m + 1) / 2 + m);
+        };
+        if (bytes((size_t)order) > (64 << 10)) {  // 133 KB at order 128 in FP64
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&trsm_dot_kernel<T>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes(128));
+            (void)hipGetLastError();
+        }
+        hipLaunchKernelGGL(trsm_dot_kernel<T>, dim3(cdiv(nvec, DNT)), dim3(256), bytes((size_t)order), s,
+                           (int)order, nvec, A, lda, B, ldb, right ? 1 : 0, unit, stop);
         ELX_HIP(hipGetLastError());
         return ELX_SUCCESS;
     }

@@ -48,3 +48,29 @@ def test_trsm_block_edges(dev, orc, side):
                         ref = orc.trsm("LR"[side], "LU"[uplo], "NT"[orient], "NU"[diag], 1.0,
                                        np.asfortranarray(T), np.asfortranarray(B))
                         assert np.array_equal(dev.to_host(dB), ref)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("order", [1, 2, 8, 33, 64, 128])
+def test_trsm_block_small_orders_and_range(dev, orc, order, dtype):
+    """Orders below and between the 16-entry blocks, vectors down to the smallest subnormals and
+    divisors far from 1."""
+    rng = np.random.default_rng(order)
+    low, high = (-1070, 500) if dtype == np.float64 else (-146, 60)
+    for other in (1, 5, 66):
+        for spread in (0, 70 if dtype == np.float32 else 450):
+            T = rng.standard_normal((order, order)) / order
+            T[np.diag_indices(order)] = np.ldexp(1 + rng.random(order), rng.integers(-spread, spread + 1, order))
+            T = T.astype(dtype)
+            for side in (0, 1):
+                V = np.ldexp(rng.standard_normal((order, other)), rng.integers(low, high, other))
+                B = (V if side == 0 else V.T).astype(dtype)
+                for uplo in (0, 1):
+                    for orient in (0, 1):
+                        for diag in (0, 1):
+                            print("[case]", dtype.__name__, order, other, spread, side, uplo, orient, diag, flush=True)
+                            dB = dev.to_device(np.ascontiguousarray(B))
+                            dev.trsm(side, uplo, orient, diag, 1.0, dev.to_device(T), dB)
+                            ref = orc.trsm("LR"[side], "LU"[uplo], "NT"[orient], "NU"[diag], 1.0,
+                                           np.asfortranarray(T), np.asfortranarray(B))
+                            assert np.array_equal(dev.to_host(dB), ref, equal_nan=True)
