@@ -25,17 +25,20 @@ namespace {
 // so the results are the scalar code's bit for bit. No workgroup barrier; the triangle is read
 // straight from the caches in operand layout. Divisions are quotients by the reciprocal where the
 // operands allow it (wave.hpp), else the block is solved again with plain ones. What bounds it: per
-// wave 8 dependent block solves of 16 steps and 28 tile products, FP64 17-27 us (right side), 11-24
-// us (left, unit diagonal) and, left and non-unit, 15 us for one vector (23 with plain divisions, 20
-// with 16 lanes per vector), one wave per SIMD; with 16 lanes per vector, all 128 steps dependent and
-// 132 KB of LDS per 16 vectors, it took 52 us per 4096 vectors (240 us at 16256).
+// wave 8 dependent block solves of 16 steps and 28 tile products, and the fetch of their straight-line
+// code: FP64 17-27 us (right side) and 11-24 us (left) from 64 to 16384 vectors, 9 us for one (left,
+// non-unit), one wave per SIMD; with 16 lanes per vector, all 128 steps dependent and 132 KB of LDS
+// per 16 vectors, it took 52 us per 4096 vectors (240 us at 16256) and 20 us for one.
 //
 // maxbits (may be null): the largest |entry| written is folded into *maxbits (the bits of a
 // non-negative float, atomic max), for the exponent of a low-precision product that follows.
 // ---------------------------------------------------------------------------------------
 constexpr int TBLK = 16, TNB = 8;  // entries per block, blocks
 // FULL: order 128, no bounds on the order (the loads are then unconditional and go out together).
-template <typename T, bool RIGHT, bool UNIT, bool FULL>
+// NR: vectors per lane, 4, or (left side) 1 where there are at most 4 vectors in all: the steps' code,
+// which a few waves fetch as they go through it once, is a quarter as long (FP64, left, non-unit, one
+// vector, launch included: order 128 25.4 -> 18.9 us, order 64 20.3 -> 17.5).
+template <typename T, bool RIGHT, bool UNIT, bool FULL, int NR>
 __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const T* __restrict__ A,
                                                          i64 lda, T* B, i64 ldb, int mtrans, int back,
                                                          const int32_t* __restrict__ stop,
@@ -58,17 +61,21 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
     const T* __restrict__ Ml = M0 + l16 * si;            // row l16 of M
     const T* __restrict__ Mk = Ml + kq * sj;             // and column kq: operand layout
     const bool vin = v0 + l16 < nvec;
-    // the vectors: LEFT D(v, i), RIGHT D(i, v), so that lanes run along the contiguous index
+    // the vectors: LEFT D(v, i), its row MF::row(kq, r) vector kq + 4 r; RIGHT D(i, v), so that lanes
+    // run along the contiguous index
     typename MF::acc acc[TNB];
 #pragma unroll
     for (int b = 0; b < TNB; ++b)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = MF::row(kq, r);
-            const int i = TBLK * b + (RIGHT ? row : l16);
-            const i64 v = v0 + (RIGHT ? l16 : row);
-            acc[b][r] = ((FULL || i < m) && (RIGHT ? vin : v < nvec)) ? X0[i * ei + v * ev] : T(0);
+            const int i = TBLK * b + (RIGHT ? MF::row(kq, r) : l16);
+            const i64 v = v0 + (RIGHT ? l16 : kq + 4 * r);
+            acc[b][r] = (r < NR && (FULL || i < m) && (RIGHT ? vin : v < nvec)) ? X0[i * ei + v * ev] : T(0);
         }
+    if (NR < 4) {  // the rows of the tile that no vector takes
+#pragma unroll
+        for (int r = NR; r < 4; ++r) tile[MF::row(kq, r)][l16] = T(0);
+    }
     float mx = 0.0f;
     // a block's triangle (row l16), diagonal and the operands M(i, k) of the later blocks, loaded
     // one block ahead
@@ -95,30 +102,30 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
         if (FULL || TBLK * b < m) {
             if constexpr (b + 1 < TNB) load(std::integral_constant<int, b + 1>{});
             const T dg = dgv[p], dr = UNIT ? T(1) : T(1) / dg;
-            // S(v, i): lane l16 holds entry i, register r vector MF::row(kq, r)
-            T x[4];
+            // S(v, i): lane l16 holds entry i, register r the vector of the tile's row MF::row(kq, r)
+            T x[NR];
             if (RIGHT) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) tile[MF::row(kq, r)][l16] = acc[b][r];
                 wave_lds_sync();
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x[r] = tile[l16][MF::row(kq, r)];
+                for (int r = 0; r < NR; ++r) x[r] = tile[l16][MF::row(kq, r)];
                 wave_lds_sync();
             } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x[r] = acc[b][r];
+                for (int r = 0; r < NR; ++r) x[r] = acc[b][r];
             }
             // a lane's entry is final (but for its own diagonal) once the earlier ones are applied;
             // every lane scales its entry at each step, and the step's own is lane k's
             auto substitute = [&](auto scale) {
                 static_for<0, TBLK>([&](auto kc) {
                     constexpr int k = decltype(kc)::value;
-                    T xk[4];
+                    T xk[NR];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) xk[r] = row_bcast<k>(scale(x[r]));
+                    for (int r = 0; r < NR; ++r) xk[r] = row_bcast<k>(scale(x[r]));
                     if (l16 > k) {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) x[r] = __builtin_fma(-mrow[p][k], xk[r], x[r]);
+                        for (int r = 0; r < NR; ++r) x[r] = __builtin_fma(-mrow[p][k], xk[r], x[r]);
                     }
                 });
             };
@@ -127,31 +134,31 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
             } else if constexpr (RIGHT) {
                 substitute([&](T v) { return v * dr; });
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x[r] = x[r] * dr;
+                for (int r = 0; r < NR; ++r) x[r] = x[r] * dr;
             } else {
                 substitute([&](T v) { return quot(v, dg, dr); });
                 bool ok = divisor_ok(dg);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ok = ok && dividend_ok(x[r]);
+                for (int r = 0; r < NR; ++r) ok = ok && dividend_ok(x[r]);
                 if (__all(ok ? 1 : 0)) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = quot(x[r], dg, dr);
+                    for (int r = 0; r < NR; ++r) x[r] = quot(x[r], dg, dr);
                 } else {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = acc[b][r];
+                    for (int r = 0; r < NR; ++r) x[r] = acc[b][r];
                     substitute([&](T v) { return v / dg; });
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = x[r] / dg;
+                    for (int r = 0; r < NR; ++r) x[r] = x[r] / dg;
                 }
             }
             if (maxbits) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, (float)fabs(x[r]));
+                for (int r = 0; r < NR; ++r) mx = fmaxf(mx, (float)fabs(x[r]));
             }
             // into operand layout: X(v = l16, k = kq + 4 kk)
             T xop[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) tile[MF::row(kq, r)][l16] = x[r];
+            for (int r = 0; r < NR; ++r) tile[MF::row(kq, r)][l16] = x[r];
             wave_lds_sync();
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) xop[kk] = tile[l16][kq + 4 * kk];
@@ -159,8 +166,11 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int m, i64 nvec, const 
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int i = TBLK * b + (RIGHT ? kq + 4 * r : l16);
-                const i64 v = v0 + (RIGHT ? l16 : MF::row(kq, r));
-                if ((FULL || i < m) && (RIGHT ? vin : v < nvec)) X0[i * ei + v * ev] = RIGHT ? xop[r] : x[r];
+                const i64 v = v0 + (RIGHT ? l16 : kq + 4 * r);
+                if ((FULL || i < m) && (RIGHT ? vin : v < nvec)) {
+                    if constexpr (RIGHT) X0[i * ei + v * ev] = xop[r];
+                    else if (r < NR) X0[i * ei + v * ev] = x[r < NR ? r : 0];
+                }
             }
             // b_i -= m_ik x_k as fma(m_ik, -x_k, b_i): the same number
 #pragma unroll
@@ -330,14 +340,21 @@ static elx_status_t trsm_small_impl(hipStream_t s, int side, int uplo, int orien
     }
     const dim3 grid(cdiv(nvec, 4 * TBLK));
     const int back = lower_eff ? 0 : 1;
-    auto go = [&](auto rt, auto ut) {
+    auto go_n = [&](auto rt, auto ut, auto nt) {
         constexpr bool R = decltype(rt)::value, U = decltype(ut)::value;
+        constexpr int N = decltype(nt)::value;
         if (order == TBLK * TNB)
-            hipLaunchKernelGGL((trsm_block_kernel<T, R, U, true>), grid, dim3(256), 0, s, (int)order,
+            hipLaunchKernelGGL((trsm_block_kernel<T, R, U, true, N>), grid, dim3(256), 0, s, (int)order,
                                nvec, A, lda, B, ldb, mt, back, stop, maxbits);
         else
-            hipLaunchKernelGGL((trsm_block_kernel<T, R, U, false>), grid, dim3(256), 0, s, (int)order,
+            hipLaunchKernelGGL((trsm_block_kernel<T, R, U, false, N>), grid, dim3(256), 0, s, (int)order,
                                nvec, A, lda, B, ldb, mt, back, stop, maxbits);
+    };
+    auto go = [&](auto rt, auto ut) {
+        if constexpr (!decltype(rt)::value) {
+            if (nvec <= 4) return go_n(rt, ut, std::integral_constant<int, 1>{});
+        }
+        go_n(rt, ut, std::integral_constant<int, 4>{});
     };
     const std::true_type yes;
     const std::false_type no;
