@@ -339,6 +339,10 @@ elx_status_t gate_slot(double** out) {
 
 namespace {
 
+// Up to as many right-hand sides a left solve is chained: 8 groups of 16, each of which reads the
+// triangle. At 128 of them the chain takes, lower non-unit FP64 (FP32), 67 (63) us at n = 200, 274
+// (237) at 1024, 807 (669) at 3001 and 2200 (1810) at 8192; block by block 129 take 91 (84), 447
+// (390), 1600 (1260) and 3750 (3240).
 constexpr i64 kChainRhs = 128;
 
 // General triangular solve: small-kernel diagonal blocks + MFMA GEMM updates. `stop` as in
@@ -357,8 +361,10 @@ elx_status_t trsm_blocked(hipStream_t s, int side, int uplo, int orient, int dia
     const bool trans = (orient != kNormal);
     const i64 bs = 128;
     // few right-hand sides: one chained launch instead of a diagonal solve and a GEMM per block
-    // (not where nothing may be allocated: its hand-off area is)
-    if (side == kLeft && allow_library && n <= kChainRhs && !(dot_order && m <= bs)) {
+    // (not where nothing may be allocated: its hand-off area is). A single block has no one to hand
+    // on to, and the small kernel takes it faster: potrs (FP64, both triangles) of order 16 with one
+    // right-hand side 38.8 -> 16.1 us, of order 128 48.2 -> 30.7, with 16 of them 61.3 -> 45.0
+    if (side == kLeft && allow_library && n <= kChainRhs && m > bs) {
         bool taken = false;
         ELX_CHECK(launch_solve_chain(s, uplo, orient, diag, m, n, A, lda, B, ldb, stop, &taken));
         if (taken) return ELX_SUCCESS;

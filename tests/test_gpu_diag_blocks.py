@@ -74,3 +74,37 @@ def test_trsm_block_small_orders_and_range(dev, orc, order, dtype):
                             ref = orc.trsm("LR"[side], "LU"[uplo], "NT"[orient], "NU"[diag], 1.0,
                                            np.asfortranarray(T), np.asfortranarray(B))
                             assert np.array_equal(dev.to_host(dB), ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 16, 17, 100, 128])
+def test_factored_solves_of_one_block(dev, orc, n, dtype):
+    """potrs and getrs of one block: the bits of their triangular solves, one after the other."""
+    rng = np.random.default_rng(n)
+    T = rng.standard_normal((n, n)) / n + 2 * np.eye(n)
+    dT, dests = dev.to_device(T.astype(dtype)), None
+    for nrhs in (1, 4, 5, 40):
+        B = rng.standard_normal((n, nrhs)).astype(dtype)
+        for name, forms in (("potrs lower", [(0, 0, 0), (0, 1, 0)]), ("potrs upper", [(1, 1, 0), (1, 0, 0)]),
+                            ("getrs", [(0, 0, 1), (1, 0, 0)])):
+            print("[case]", dtype.__name__, n, nrhs, name, flush=True)
+            got, wide = dev.to_device(B), np.zeros((n, 130), dtype)
+            wide[:, :nrhs] = B
+            one = dev.to_device(wide)
+            if name == "getrs":
+                dev.getrs(dT, dests, got)
+                dev.getrs(dT, dests, one)
+            else:
+                dev.potrs(dT, got, uplo=forms[0][0])
+                dev.potrs(dT, one, uplo=forms[0][0])
+            x = dev.to_host(got)
+            assert np.array_equal(x, dev.to_host(one)[:, :nrhs])
+            r = B.astype(np.float64)
+            for uplo, orient, diag in reversed(forms):
+                M = np.tril(T) if uplo == 0 else np.triu(T)
+                M = M.astype(dtype).astype(np.float64)
+                if diag:
+                    M = M - np.diag(np.diag(M)) + np.eye(n)
+                x = (M.T if orient else M) @ x
+            u = np.finfo(dtype).eps / 2
+            assert np.abs(x - r).max() <= 64 * n * u * np.abs(r).max()
