@@ -2,6 +2,7 @@
 one FMA chain over ascending k, so it equals the same columns of a wider product bit for bit."""
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -23,3 +24,35 @@ def test_narrow_equals_wide(dev, dtype, alpha):
                 dev.gemm(0, 0, alpha, dA, dB[:, :n], 1.0, part[:, :n])
                 assert np.array_equal(dev.to_host(part)[:, :n], dev.to_host(wide)[:, :n])
                 assert np.array_equal(dev.to_host(part)[:, n:], C[:, n:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 5), (100, 4000, 7), (130, 1500, 33), (2100, 129, 50), (127, 300, 64),
+                                   (1300, 1300, 17), (1500, 1500, 127)])
+def test_every_tile_of_a_ragged_product(dev, m, n, k, dtype):
+    """No whole tile (K not a multiple of 16, or C smaller than one): whole-number operands, so the
+    product is exact in any order, and every entry of C, inside the triangle only for syrk."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+
+    def ints(a, b):
+        t = dev.colmajor_empty(a, b, dtype)
+        t.copy_(torch.randint(-8, 9, (a, b), device="cuda", generator=g))
+        return t
+
+    for ta in (0, 1):
+        for tb in (0, 1):
+            print("[case]", m, n, k, dtype, ta, tb, flush=True)
+            A, B, C = ints(*((k, m) if ta else (m, k))), ints(*((n, k) if tb else (k, n))), ints(m, n)
+            want = C.cpu().double() - (A.t() if ta else A).cpu().double() @ (B.t() if tb else B).cpu().double()
+            dev.gemm(ta, tb, -1.0, A, B, 1.0, C)
+            assert torch.equal(C.cpu().double(), want)
+        if m == n:
+            for uplo in (0, 1):
+                A, C = ints(*((k, m) if ta else (m, k))), ints(m, m)
+                P = (A.t() if ta else A).cpu().double()
+                full = C.cpu().double()
+                mask = torch.ones(m, m).tril() if uplo == 0 else torch.ones(m, m).triu()
+                want = torch.where(mask > 0, full - P @ P.t(), full)
+                dev.syrk(uplo, ta, -1.0, A, 1.0, C)
+                assert torch.equal(C.cpu().double(), want)
