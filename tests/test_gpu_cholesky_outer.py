@@ -27,12 +27,17 @@ def colmajor(dev, a, pad):
     return t
 
 
+# Orders with one outer block and with two, one after the other (both start with at least 8192 rows left).
+# Stops in the first, a later and the last panel of an outer block and behind the last outer block.
 @pytest.mark.parametrize("uplo", [0, 1])
-@pytest.mark.parametrize("n,pad", [(8192, 0), (8300, 1)])
-def test_outer_blocks(dev, n, pad, uplo, dtype=torch.float64):
+@pytest.mark.parametrize("n,pad,fails", [
+    (8192, 0, (10, 2 * 128 + 10, 8192 - 10, 8192 - 256 + 10)),
+    (8300, 1, (10, 2 * 128 + 10, 8300 - 10, 63 * 128 + 10)),
+    (8748, 0, (3 * 128 + 10, 512 + 10, 512 + 128 + 10, 512 + 384 + 10, 1024 + 10)),
+])
+def test_outer_blocks(dev, n, pad, fails, uplo, dtype=torch.float64):
     H = hpd(n, dtype, n)
-    # a clean factorization, and stops in the first and a later panel of an outer block
-    for fail in (None, 10, 2 * 128 + 10, n - 10):
+    for fail in (None,) + fails:
         print("[case]", n, pad, uplo, fail, flush=True)
         A = H.clone()
         if fail is not None:
@@ -40,14 +45,18 @@ def test_outer_blocks(dev, n, pad, uplo, dtype=torch.float64):
         a, b = colmajor(dev, A, pad), colmajor(dev, A, pad)
         ia, ib = dev.potrf(a, uplo=uplo, nb=128), dev.potrf(b, uplo=uplo, nb=64)
         assert int(ia.item()) == int(ib.item()) == (0 if fail is None else fail + 1)
-        # right of the failing 128-column panel (the panel itself stops at a block edge of its own)
-        c = 0 if fail is None else fail // 128 * 128 + 128
+        # the columns finished before the failing 128-column panel and those right of it (the panel itself
+        # stops at a block edge of its own)
+        p, c = (n, n) if fail is None else (fail // 128 * 128, fail // 128 * 128 + 128)
         if fail is not None and fail % 128 >= 64:
             continue  # the 64-column blocks complete half a panel more
         x, y = (a.t(), b.t()) if uplo == 0 else (a, b)  # row j: the entries of column (row) j
-        if uplo == 0:
-            assert torch.equal(x[c:, c:], y[c:, c:])
-        else:
-            x, y = x[c:, c:], y[c:, c:]
-            if y.numel():
-                assert float((x - y).abs().max()) <= 8 * n * 2.0 ** -53 * float(y.abs().max())
+        assert fail is None or c < n
+        for part in (slice(0, p), slice(c, n)):
+            u, v = x[part], y[part]
+            if u.numel() == 0:
+                continue
+            if uplo == 0:
+                assert torch.equal(u, v)
+            else:
+                assert float((u - v).abs().max()) <= 8 * n * 2.0 ** -53 * float(v.abs().max())
