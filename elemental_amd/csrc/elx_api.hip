@@ -583,12 +583,16 @@ elx_status_t potrf_impl(hipStream_t s, int uplo, i64 n, T* A, i64 lda, i64 nb, i
         if (n2 > 0) {
             T* P = lower ? A + kend + k0 * lda : A + k0 + kend * lda;
             T* C = A + kend + kend * lda;
-            if (deep)
-                ELX_CHECK(launch_gemm_from(s, !lower, lower, n2, n2, d, T(-1), P, lda, P, lda, T(1), C, lda,
-                                           lower ? 1 : 2, info, k0));
-            else
-                ELX_CHECK(launch_gemm(s, !lower, lower, n2, n2, d, T(-1), P, lda, P, lda, T(1), C, lda,
-                                      lower ? 1 : 2, info));
+            if constexpr (sizeof(T) == 8) {
+                if (deep) {
+                    ELX_CHECK(launch_gemm_from(s, !lower, lower, n2, n2, d, T(-1), P, lda, P, lda, T(1), C, lda,
+                                               lower ? 1 : 2, info, k0));
+                    k0 = kend;
+                    continue;
+                }
+            }
+            ELX_CHECK(launch_gemm(s, !lower, lower, n2, n2, d, T(-1), P, lda, P, lda, T(1), C, lda,
+                                  lower ? 1 : 2, info));
         }
         k0 = kend;
     }

@@ -175,9 +175,6 @@ elx_status_t gate_slot(double** out);
 elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, double alpha,
                               const double* A, i64 lda, const double* B, i64 ldb, double beta,
                               double* C, i64 ldc, int tri, const int32_t* stop, i64 from);
-elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, float alpha,
-                              const float* A, i64 lda, const float* B, i64 ldb, float beta, float* C,
-                              i64 ldc, int tri, const int32_t* stop, i64 from);
 bool gemm_library_selected();  // ELX_DGEMM=library
 
 // Small triangular solves for many independent vectors (triangle order <= 128).

@@ -709,13 +709,6 @@ elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64
     return gemm_impl<double>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri, stop, false,
                              from);
 }
-elx_status_t launch_gemm_from(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, float alpha,
-                              const float* A, i64 lda, const float* B, i64 ldb, float beta, float* C,
-                              i64 ldc, int tri, const int32_t* stop, i64 from) {
-    return gemm_impl<float>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri, stop, false,
-                            from);
-}
-
 elx_status_t launch_dgemm(hipStream_t s, bool ta, bool tb, i64 m, i64 n, i64 k, double alpha,
                           const double* A, i64 lda, const double* B, i64 ldb, double beta,
                           double* C, i64 ldc, int tri) {

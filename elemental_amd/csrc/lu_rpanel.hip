@@ -37,6 +37,9 @@ using elx::xchg::ld16;
 using elx::xchg::mix32;
 using elx::xchg::st16;
 using elx::xchg::u4;
+using elx::wv::bcast_lane;
+using elx::wv::row_bcast;
+using elx::wv::static_for;
 
 constexpr int NTMAX = 512;                 // 8 waves: two per SIMD, 256 VGPRs each
 constexpr int WS = 32;                     // columns per block
@@ -124,25 +127,6 @@ __device__ __forceinline__ int wave_argmax(Key k, uint32_t lbl) {
     return __ffsll((unsigned long long)hit) - 1;
 }
 
-// Entry J of a row held one entry per lane (repeated in every 16-lane row), in every lane.
-template <int J>
-__device__ __forceinline__ double bcast(double v) {
-    return __longlong_as_double(
-        __builtin_amdgcn_update_dpp(0LL, (long long)__double_as_longlong(v), 0x150 + J, 0xF, 0xF, true));
-}
-template <int J>
-__device__ __forceinline__ float bcast(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + J, 0xF, 0xF, true));
-}
-
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
 __device__ __forceinline__ void bits_of(double v, uint32_t& lo, uint32_t& hi) {
     const uint64_t b = (uint64_t)__double_as_longlong(v);
     lo = (uint32_t)b;
@@ -156,16 +140,6 @@ __device__ __forceinline__ void value_of(u4 c, double& v) {
     v = __longlong_as_double((long long)(((uint64_t)c[1] << 32) | c[0]));
 }
 __device__ __forceinline__ void value_of(u4 c, float& v) { v = __uint_as_float(c[0]); }
-
-// The value of lane k in every lane (k uniform).
-__device__ __forceinline__ double lane_val(double v, int k) {
-    uint32_t lo, hi;
-    bits_of(v, lo, hi);
-    return __hiloint2double(__builtin_amdgcn_readlane((int)hi, k), __builtin_amdgcn_readlane((int)lo, k));
-}
-__device__ __forceinline__ float lane_val(float v, int k) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
-}
 
 __device__ __forceinline__ uint32_t xcc_id() {
     uint32_t x;
@@ -406,7 +380,7 @@ __global__ __launch_bounds__(NT) void rpanel_kernel(RArgs<T> p) {
                     T ub[8];
                     static_for<e0, 8>([&](auto ec) {
                         constexpr int e = decltype(ec)::value, j = 8 * k + e;
-                        ub[e] = bcast<j & 15>(j < 16 ? u0 : u1);
+                        ub[e] = row_bcast<j & 15>(j < 16 ? u0 : u1);
                     });
                     static_for<0, RPT>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
@@ -513,7 +487,7 @@ __global__ __launch_bounds__(256) void panel_solve_kernel(T* P, i64 lda, i64 mp,
             if (k < steps) {
 #pragma unroll
                 for (int q = 0; q < CW; ++q) {
-                    const T xk = lane_val(x[q], k);
+                    const T xk = bcast_lane(x[q], k);
                     if (lane < 32 && lane > k) x[q] = __builtin_fma(-l[k], xk, x[q]);
                 }
             }
