@@ -339,11 +339,18 @@ elx_status_t gate_slot(double** out) {
 
 namespace {
 
-// Up to as many right-hand sides a left solve is chained: 8 groups of 16, each of which reads the
-// triangle. At 128 of them the chain takes, lower non-unit FP64 (FP32), 67 (63) us at n = 200, 274
-// (237) at 1024, 807 (669) at 3001 and 2200 (1810) at 8192; block by block 129 take 91 (84), 447
-// (390), 1600 (1260) and 3750 (3240).
-constexpr i64 kChainRhs = 128;
+// Whether a left solve of order m > 128 is chained: up to 128 right-hand sides, 8 groups of 16, each
+// of which reads the triangle. At 128 of them the chain and the blocks take (lower, non-unit, FP64)
+// 59 and 80 us at m = 200, 236 and 368 at 1024, 684 and 1430 at 3001, 1990 and 3120 at 8192, 5810 and
+// 6450 at 16384, 11.8 and 9.9 ms at 24576, 19.6 and 13.5 at 32768; in FP32 51 and 70, 187 and 280, 513
+// and 1080, 1370 and 2290, 3150 and 4720 us, 6.0 and 7.2, 9.7 and 9.8 ms. What the groups read grows
+// with m^2, a step of the blocked solve stays at 35 to 60 us per 128 rows: the line lies at 7 groups of
+// 24576 rows in FP64 (10.5 and 11.1 ms; 6 of 32768 15.3 and 14.9, 5 of them 13.4 and 14.8).
+template <typename T>
+bool chain_pays(i64 m, i64 nrhs) {
+    const i64 groups = (nrhs + 15) / 16;
+    return m > 128 && groups <= 8 && groups * m * (i64)sizeof(T) <= 7 * 24576 * (i64)sizeof(double);
+}
 
 // General triangular solve: small-kernel diagonal blocks + MFMA GEMM updates. `stop` as in
 // the launchers: a recorded failure makes every step a no-op. allow_library false keeps the
@@ -364,7 +371,7 @@ elx_status_t trsm_blocked(hipStream_t s, int side, int uplo, int orient, int dia
     // (not where nothing may be allocated: its hand-off area is). A single block has no one to hand
     // on to, and the small kernel takes it faster: potrs (FP64, both triangles) of order 16 with one
     // right-hand side 38.8 -> 16.1 us, of order 128 48.2 -> 30.7, with 16 of them 61.3 -> 45.0
-    if (side == kLeft && allow_library && n <= kChainRhs && m > bs) {
+    if (side == kLeft && allow_library && chain_pays<T>(m, n)) {
         bool taken = false;
         ELX_CHECK(launch_solve_chain(s, uplo, orient, diag, m, n, A, lda, B, ldb, stop, &taken));
         if (taken) return ELX_SUCCESS;

@@ -11,9 +11,10 @@
 // rows at a time: wave w holds rows 16 w .. 16 w + 15 of all 16 vectors in one MFMA accumulator,
 // wave s solves its 16 x 16 triangle, and the waves below it update on the matrix cores. What
 // bounds it is that chain per block: 8 dependent 16-row solves, and the hand-off of the block's
-// solution through memory, 18 us (unit diagonal) to 24 us (up to 4 vectors) and 35 us (5 to 16)
-// together; the matrix is read once, half a tile ahead. n = 16384: 15 -> 3.2 ms per triangle with
-// one right-hand side, 8.9 -> 4.4 ms with 16; n = 1024: 0.52 -> 0.19 ms.
+// solution through memory, in FP64 (FP32) 19 (12) us with a unit diagonal, 21 (14) without one, 28 (21)
+// for 5 to 16 vectors; the matrix is read once, half a tile ahead. FP64, per triangle, the pairs of kernels
+// before -> this one: n = 16384 15 -> 2.7 ms with one right-hand side, 8.9 -> 3.6 ms with 16; n = 1024
+// 0.52 -> 0.18 ms.
 //
 // Every entry is updated in the order of the blocked substitution: block by block, one FMA per
 // unknown of an earlier block in ascending column order, then the steps of its own block; the

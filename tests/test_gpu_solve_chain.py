@@ -257,3 +257,23 @@ def test_divisions_at_the_ends_of_the_range(dev, dtype):
                 same = (x.view(bits) == y.view(bits)) | (np.isnan(x) & np.isnan(y))
                 print("[case]", dtype.__name__, spread, orient, cols, int((~same).sum()), flush=True)
                 assert same.all()
+
+
+def test_many_columns_of_a_large_order(dev):
+    """128 columns of an order past the chained solve's range are solved block by block, to the bits of
+    the chained solve of 16 of them."""
+    n = 24576
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    dT = dev.colmajor_empty(n, n)
+    torch.randn(n, n, dtype=torch.float64, device="cuda", generator=g, out=dT.t())
+    dT.mul_(1.0 / n)
+    dT.diagonal().add_(1.0)
+    B = torch.randn(n, 128, dtype=torch.float64, device="cuda", generator=g)
+    for uplo in (0, 1):
+        wide, part = dev.colmajor_empty(n, 128), dev.colmajor_empty(n, 16)
+        wide.copy_(B)
+        part.copy_(B[:, 64:80])
+        dev.trsm(0, uplo, 0, 0, 1.0, dT, wide)
+        dev.trsm(0, uplo, 0, 0, 1.0, dT, part)
+        assert torch.equal(wide[:, 64:80], part)
