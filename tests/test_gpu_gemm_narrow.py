@@ -28,10 +28,12 @@ def test_narrow_equals_wide(dev, dtype, alpha):
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 5), (100, 4000, 7), (130, 1500, 33), (2100, 129, 50), (127, 300, 64),
-                                   (1300, 1300, 17), (1500, 1500, 127)])
+                                   (1152, 1152, 64), (1300, 1300, 17), (1500, 1500, 127), (2100, 2100, 33),
+                                   (3200, 3200, 16)])
 def test_every_tile_of_a_ragged_product(dev, m, n, k, dtype):
-    """No whole tile (K not a multiple of 16, or C smaller than one): whole-number operands, so the
-    product is exact in any order, and every entry of C, inside the triangle only for syrk."""
+    """Grids without whole tiles (K not a multiple of 16, or C smaller than one), and triangles whose
+    last group of 8 tile rows has 1, 3, 4 or 8: whole-number operands, so the product is exact in any
+    order, and every entry of C, inside the triangle only for syrk."""
     g = torch.Generator(device="cuda")
     g.manual_seed(m + n + k)
 
