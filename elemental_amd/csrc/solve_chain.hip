@@ -127,12 +127,13 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
     auto vcol = [&](int r) { return kq + 4 * r; };
     bool lost = false;
 
+    const int items = nblk * p.groups;
     for (;;) {
         // the next block, the groups of right-hand sides side by side
         if (t == 0) s_item = atomicAdd(&p.ctrl[2], 1u);
         __syncthreads();
         const int item = __builtin_amdgcn_readfirstlane((int)s_item);
-        if (item >= nblk * p.groups) break;
+        if (item >= items) break;
         const int b = item / p.groups, group = item - b * p.groups;
         const i64 v0 = (i64)group * NV;
         const int nv = (int)((p.nrhs - v0) < NV ? (p.nrhs - v0) : NV);
@@ -321,6 +322,7 @@ __global__ __launch_bounds__(CNT) void solve_chain_kernel(ChainArgs<T> p) {
             const int i = idx & (BS - 1), v = idx >> 7;
             if (i0 + i >= lo && i0 + i < hi && v < nv) X0[(i0 + i) * ei + v * p.ldb] = xd[i][v];
         }
+        if (item == items - 1) break;  // the launch ends with this block: it does not ask for another
         __syncthreads();
     }
     // the last workgroup to finish opens the next launch's epoch and its count of blocks, and reports a
