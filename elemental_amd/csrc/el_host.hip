@@ -344,11 +344,11 @@ Int blocksize_checked() {
 }
 
 // The info word of a device factorization as the reference reports it: 0 success, j+1 the
-// first failing column (the caller throws its exception), and -1 (the device panel gave up
-// waiting for a peer workgroup) a runtime error.
+// first failing column (the caller throws its exception), and -1 (the device panel, or the solve
+// behind it, gave up waiting for a peer workgroup) a runtime error.
 int read_info_checked(const DevBuf& info, const char* what) {
     const int v = read_info(info);
-    if (v < 0) RuntimeError(std::string(what) + ": device panel did not complete");
+    if (v < 0) RuntimeError(std::string(what) + ": device kernel did not complete");
     return v;
 }
 

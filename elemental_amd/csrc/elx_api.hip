@@ -81,7 +81,7 @@ elx_status_t coop_fits(const void* fn, int block, size_t lds, i64 grid) {
     ELX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, block, lds));
     if (grid > (i64)per_cu * di.num_cus) {
         std::fprintf(stderr,
-                     "elemental_amd: cooperative launch of %lld workgroups exceeds %d per CU x %d "
+                     "elemental_amd: launch of %lld workgroups that wait for each other exceeds %d per CU x %d "
                      "CUs\n",
                      (long long)grid, per_cu, di.num_cus);
         return ELX_ERROR_NOT_SUPPORTED;

@@ -159,7 +159,7 @@ def test_trsm_many_rhs_blocked_bitwise(dev, orc, dtype):
 
 
 def test_lu_single_panel_bitwise(dev, orc):
-    """n <= nb (and tall single panels: one cooperative panel over many workgroups) runs only
+    """n <= nb (and tall single panels: one panel over many workgroups) runs only
     the panel kernel, whose per-entry FMA order is lu::Panel's: the factors are asserted equal
     to the oracle's bit for bit."""
     orc.rng_seed(17)
