@@ -2,6 +2,7 @@
 it stops, and beside infinities) and triangular solves of order <= 128, bit for bit the oracle's."""
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +109,28 @@ def test_factored_solves_of_one_block(dev, orc, n, dtype):
                 x = (M.T if orient else M) @ x
             u = np.finfo(dtype).eps / 2
             assert np.abs(x - r).max() <= 64 * n * u * np.abs(r).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_trsm_block_under_capture(dev, dtype):
+    """The order-128 forms captured and replayed, eager solves between the replays."""
+    rng = np.random.default_rng(3)
+    dT = dev.to_device((rng.standard_normal((128, 128)) / 128 + 2 * np.eye(128)).astype(dtype))
+    B = torch.from_numpy(rng.standard_normal((128, 70)).astype(dtype)).cuda()
+    forms = [(uplo, orient, diag) for uplo in (0, 1) for orient in (0, 1) for diag in (0, 1)]
+    outs = [dev.colmajor_empty(128, 70, B.dtype) for _ in forms]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for out, (uplo, orient, diag) in zip(outs, forms):
+            dev.trsm(0, uplo, orient, diag, 1.0, dT, out)
+    for _ in range(3):
+        for out in outs:
+            out.copy_(B)
+        g.replay()
+        torch.cuda.synchronize()
+        for out, (uplo, orient, diag) in zip(outs, forms):
+            eager = dev.colmajor_empty(128, 70, B.dtype)
+            eager.copy_(B)
+            dev.trsm(0, uplo, orient, diag, 1.0, dT, eager)
+            assert torch.equal(out, eager)
